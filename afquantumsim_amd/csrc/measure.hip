@@ -28,6 +28,7 @@ namespace {
 constexpr int kBlock = 256;
 static_assert(kBlock == 256, "the block reductions combine four waves");
 constexpr int kRedGrid = 1024;       // fixed reduction grid (deterministic order)
+constexpr uint64_t kOneBlockUnits = 4096;
 constexpr int kSampleBlock = 1024;   // amplitudes per sampling block
 constexpr double kFixScale = 1152921504606846976.0;  // 2^60
 
@@ -158,6 +159,106 @@ __global__ __launch_bounds__(kBlock) void k_reduce(const T2* __restrict__ a, uin
     if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = r;
     __syncthreads();
     if (threadIdx.x == 0) partial[blockIdx.x] = (sh[0] + sh[1]) + (sh[2] + sh[3]);
+}
+
+// P(q = 1) of every qubit in one sweep.  A workgroup owns `per` consecutive
+// chunks (a power of two) of 256 x kP1Units 16-byte units, so each index bit
+// is one of: the amplitude inside a unit, the thread, the unit's number in
+// the chunk, the chunk's number in the workgroup's range, or the workgroup.
+// Per amplitude only |a|^2 and the sums for the first and third kind are
+// formed; a thread's chunk sum is added once per set bit of the chunk's
+// number (uniform tests), the thread's own bits select its total when the
+// workgroup is done, the workgroup's bits select in k_prob1_final.  Sums are
+// FP64 in a fixed order.  Bound by HBM: one read of the state where one
+// reduction per qubit took n (27 qubits complex64, with <sum Z> and 1000
+// shots after it: 4992 -> 557 us, three reads of 1 GiB at 6.5 TB/s being 495).
+// At most kP1Grid workgroups: their partials fit the state's scratch at
+// every size (21 qubits: 13 values x 512 x 8 B = 52 KiB of 96).
+constexpr int kP1Units = 8;
+constexpr int kP1Grid = 512;
+constexpr int kP1LoopBits = AQS_MAX_QUBITS - 11 - 9;  // complex128 chunks hold 2^11 amplitudes
+constexpr int kP1Values = 1 + 12 + kP1LoopBits;
+
+template <typename T2>
+__global__ __launch_bounds__(kBlock) void k_prob1_all(const T2* __restrict__ a, uint64_t N, uint32_t per,
+                                                      double* __restrict__ partial) {
+    __shared__ double sh[kP1Values][kBlock / 64];
+    constexpr int A = sizeof(T2) == 8 ? 2 : 1;
+    constexpr int U = kP1Units;
+    const float4* av = reinterpret_cast<const float4*>(a);
+    const uint64_t NV = N / A;
+    double tot = 0.0, odd = 0.0, pj[3] = {0.0, 0.0, 0.0}, loop[kP1LoopBits];
+#pragma unroll
+    for (int b = 0; b < kP1LoopBits; ++b) loop[b] = 0.0;
+    for (uint32_t i = 0; i < per; ++i) {
+        const uint64_t k0 = ((uint64_t)blockIdx.x * per + i) * (kBlock * U) + threadIdx.x;
+        float4 v[U];
+#pragma unroll
+        for (int j = 0; j < U; ++j) {
+            const uint64_t k = k0 + (uint64_t)j * kBlock;
+            v[j] = k < NV ? ld_nt(&av[k]) : make_float4(0.f, 0.f, 0.f, 0.f);
+        }
+        double s[U];
+#pragma unroll
+        for (int j = 0; j < U; ++j) {
+            if (A == 2) {
+                const double q = prob_of(make_float2(v[j].z, v[j].w));
+                odd += q;
+                s[j] = prob_of(make_float2(v[j].x, v[j].y)) + q;
+            } else {
+                double2 d;
+                __builtin_memcpy(&d, &v[j], sizeof(d));
+                s[j] = prob_of(d);
+            }
+        }
+        pj[0] += (s[1] + s[3]) + (s[5] + s[7]);
+        pj[1] += (s[2] + s[3]) + (s[6] + s[7]);
+        const double hi = (s[4] + s[5]) + (s[6] + s[7]);
+        pj[2] += hi;
+        const double c = ((s[0] + s[1]) + (s[2] + s[3])) + hi;
+        tot += c;
+#pragma unroll
+        for (int b = 0; b < kP1LoopBits; ++b)
+            if ((i >> b) & 1u) loop[b] += c;
+    }
+    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    int n = 0;  // value 0: the total, value 1 + b: index bit b
+    auto put = [&](double x) {
+        const double r = wave_sum(x);
+        if (lane == 0) sh[n][w] = r;
+        ++n;
+    };
+    put(tot);
+    if (A == 2) put(odd);
+#pragma unroll
+    for (int b = 0; b < 8; ++b) put(((threadIdx.x >> b) & 1u) ? tot : 0.0);
+#pragma unroll
+    for (int j = 0; j < 3; ++j) put(pj[j]);
+#pragma unroll
+    for (int b = 0; b < kP1LoopBits; ++b)
+        if ((per >> b) > 1u) put(loop[b]);
+    __syncthreads();
+    if ((int)threadIdx.x < n) {
+        const double* r = sh[threadIdx.x];
+        partial[(uint64_t)threadIdx.x * gridDim.x + blockIdx.x] = (r[0] + r[1]) + (r[2] + r[3]);
+    }
+}
+
+// Workgroup q: P(qubit q = 1) from the partials of `grid` workgroups, each
+// covering 2^own index bits.
+__global__ __launch_bounds__(kBlock) void k_prob1_final(const double* __restrict__ partial, uint32_t grid, int own, int n,
+                                                        double* __restrict__ out) {
+    __shared__ double sh[kBlock];
+    const int b = n - 1 - (int)blockIdx.x;
+    double acc = 0.0;
+    for (uint32_t i = threadIdx.x; i < grid; i += kBlock) {
+        if (b < own)
+            acc += partial[(uint64_t)(1 + b) * grid + i];
+        else if ((i >> (b - own)) & 1u)
+            acc += partial[i];
+    }
+    const double r = block_reduce_sum(acc, sh);
+    if (threadIdx.x == 0) out[blockIdx.x] = r;
 }
 
 // <a|b> = sum conj(a_i) b_i
@@ -514,28 +615,38 @@ void launch_sampling(const void* amps, int precision, uint64_t N, const SampleTa
 }
 
 double* partial_buf(aqs_state s) { return (double*)s->scratch; }
-double* result_buf(aqs_state s) { return (double*)s->scratch + 2 * kRedGrid; }
+
+// Results of a reduction: the last kernel writes them straight into the
+// state's pinned host buffer, read after the stream is done (a copy from
+// device memory was one more command per call).
+double* result_buf(aqs_state s, int w) {
+    ensure_pinned(s, sizeof(double) * w);
+    return (double*)s->pinned;
+}
 
 void read_results(aqs_state s, double* out, int w) {
-    ensure_pinned(s, sizeof(double) * w);
-    AQS_HIP(hipMemcpyAsync(s->pinned, result_buf(s), sizeof(double) * w, hipMemcpyDeviceToHost, s->stream));
     AQS_HIP(hipStreamSynchronize(s->stream));
     std::copy((double*)s->pinned, (double*)s->pinned + w, out);
 }
 
 template <int MODE>
 double reduce_mode(aqs_state s, uint64_t mask) {
-    const unsigned g = red_grid(s->N);
+    // a state of at most kOneBlockUnits 16-byte units is summed by one
+    // workgroup in one launch
+    const uint64_t units = s->precision == AQS_C64 ? s->N / 2 : s->N;
+    const unsigned g = units <= kOneBlockUnits ? 1 : red_grid(s->N);
+    double* res = result_buf(s, 1);
+    double* part = g == 1 ? res : partial_buf(s);
     {
         ProfScope ps(s, 0);
         if (s->precision == AQS_C64)
             hipLaunchKernelGGL((k_reduce<float2, MODE>), dim3(g), dim3(kBlock), 0, s->stream, (const float2*)s->amps, s->N,
-                               mask, s->n, partial_buf(s));
+                               mask, s->n, part);
         else
             hipLaunchKernelGGL((k_reduce<double2, MODE>), dim3(g), dim3(kBlock), 0, s->stream, (const double2*)s->amps,
-                               s->N, mask, s->n, partial_buf(s));
-        hipLaunchKernelGGL(k_reduce_final, dim3(1), dim3(kBlock), 0, s->stream, (const double*)partial_buf(s), (int)g, 1,
-                           result_buf(s));
+                               s->N, mask, s->n, part);
+        if (g > 1)
+            hipLaunchKernelGGL(k_reduce_final, dim3(1), dim3(kBlock), 0, s->stream, (const double*)part, (int)g, 1, res);
         AQS_HIP(hipGetLastError());
     }
     double r;
@@ -622,10 +733,29 @@ aqs_status aqs_prob1(aqs_state s, int qubit, double* out) {
 aqs_status aqs_prob1_all(aqs_state s, double* out) {
     return guard([&] {
         check(s);
-        for (int q = 0; q < s->n; ++q) {
-            double r = reduce_mode<1>(s, qbit(s->n, q));
-            if (out) out[q] = r;
+        const int chunk_bits = s->precision == AQS_C64 ? 12 : 11;
+        const uint64_t chunks = s->n > chunk_bits ? s->N >> chunk_bits : 1;
+        const uint32_t g = (uint32_t)std::min<uint64_t>(chunks, kP1Grid);
+        const uint32_t per = (uint32_t)(chunks / g);
+        const int own = chunk_bits + __builtin_ctz(per);
+        if ((size_t)(1 + own) * g * sizeof(double) > s->scratch_bytes)
+            fail(AQS_ERR_RUNTIME, "reduction scratch too small");
+        double* res = result_buf(s, s->n);
+        {
+            ProfScope ps(s, 0);
+            if (s->precision == AQS_C64)
+                hipLaunchKernelGGL(k_prob1_all<float2>, dim3(g), dim3(kBlock), 0, s->stream, (const float2*)s->amps, s->N,
+                                   per, partial_buf(s));
+            else
+                hipLaunchKernelGGL(k_prob1_all<double2>, dim3(g), dim3(kBlock), 0, s->stream, (const double2*)s->amps,
+                                   s->N, per, partial_buf(s));
+            hipLaunchKernelGGL(k_prob1_final, dim3((unsigned)s->n), dim3(kBlock), 0, s->stream,
+                               (const double*)partial_buf(s), g, own, s->n, res);
+            AQS_HIP(hipGetLastError());
         }
+        std::vector<double> r(s->n);
+        read_results(s, r.data(), s->n);
+        if (out) std::copy(r.begin(), r.end(), out);
     });
 }
 
@@ -771,7 +901,7 @@ aqs_status aqs_inner(aqs_state a, aqs_state b, double* re_im) {
             hipLaunchKernelGGL((k_inner<double2, double2>), dim3(g), dim3(kBlock), 0, a->stream,
                                (const double2*)a->amps, (const double2*)b->amps, a->N, part);
         hipLaunchKernelGGL(k_reduce_final, dim3(1), dim3(kBlock), 0, a->stream, (const double*)part, (int)g, 2,
-                           result_buf(a));
+                           result_buf(a, 2));
         AQS_HIP(hipGetLastError());
         double r[2];
         read_results(a, r, 2);

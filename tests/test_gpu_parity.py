@@ -496,6 +496,25 @@ def test_measurement_reductions(precision):
 
 
 @pytest.mark.parametrize("precision", [hip.C64, hip.C128], ids=["c64", "c128"])
+@pytest.mark.parametrize("n", [1, 2, 8, 11, 12, 13, 14, 19, 20, 21, 23])
+def test_prob1_all_sizes(n, precision):
+    """P(q = 1) of every qubit in one sweep, at the edges of its chunks (2^12
+    or 2^11 amplitudes), of one chunk per workgroup (2^21, 2^20) and beyond,
+    against numpy and the one-qubit reduction.  FP64 sums of at most 2^23
+    terms in trees and runs of at most 2^8: far below 1e-13."""
+    st = hip.State(n, precision)
+    st.gaussian(n)
+    p = np.abs(st.download().astype(np.complex128)) ** 2
+    got = st.prob1_all()
+    index = np.arange(1 << n)
+    want = [p[(index >> (n - 1 - q)) & 1 == 1].sum() for q in range(n)]
+    np.testing.assert_allclose(got, want, rtol=0, atol=1e-13)
+    for q in {0, n // 2, n - 1}:
+        assert abs(st.prob1(q) - got[q]) < 1e-13
+    st.close()
+
+
+@pytest.mark.parametrize("precision", [hip.C64, hip.C128], ids=["c64", "c128"])
 def test_measure_qubit_collapse(precision):
     """Qubit n-1 (bit 0) splits each 16-byte pair of complex64 amplitudes
     between kept and zeroed; the zeroed ones are exactly +0."""

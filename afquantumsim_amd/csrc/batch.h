@@ -1,4 +1,4 @@
-// Batched states: the per-state program the persistent batch kernel runs
+// Batched states: the per-state program the batch kernel runs
 // (batch.hip), shared with the host emulation of the CPU tests.
 #ifndef AQS_BATCH_H
 #define AQS_BATCH_H

@@ -1,18 +1,25 @@
-// Batched simulation of many small, independent states in one persistent
+// Batched simulation of many small, independent states in one graph
 // launch (variational ansatz workload: thousands of 10-16 qubit circuits,
 // each followed by <sum Z> in FP64).
 //
 // The reference simulates one state at a time with a 2^n x 2^n operator per
-// gate (src/quantum.cpp:277-291).  Here every workgroup of a persistent grid
-// takes the next state from an atomic queue (states sorted by descending
-// cost).  A state that fits the LDS tile (2^lds_qubits amplitudes) is built
-// as |0..0> in LDS, runs all its gate passes there with a workgroup barrier
-// between passes, and is written to HBM once.  A larger state runs as a few
+// gate (src/quantum.cpp:277-291).  Here a workgroup runs one phase of one
+// tile.  A state that fits the LDS tile (2^lds_qubits amplitudes) is one tile
+// with one phase: built as |0..0> in LDS, all its gates there with a workgroup
+// barrier between segments, written to HBM once.  A larger state runs as a few
 // phases (batch_phases): per phase every tile of 2^lds_qubits amplitudes is
 // loaded into LDS, runs all of the phase's gates and is stored, so the state
-// crosses the memory hierarchy once per phase instead of once per gate.
-// <sum_q Z_q> is reduced in FP64 from the final tiles.  The launch (queue
-// reset + persistent kernel) is captured once into a hipGraph and replayed.
+// crosses the memory hierarchy once per phase instead of once per gate.  All
+// states' p-th phases are one launch (level p), one workgroup per tile, states
+// in descending order of cost.  <sum_q Z_q> is reduced in FP64 per final tile
+// and summed per state in tile order.  The launches are captured once into a
+// hipGraph and replayed.
+//
+// Why levels: one workgroup per state (a persistent grid over a queue, phases
+// and tiles in sequence inside it) left a batch waiting for its few largest
+// states, whose 8 tiles ran one after another on one of 256 CUs.  512 ansatz
+// states of 10..16 qubits: 3.12 -> 1.13 ms per run; a burst of 24 served
+// requests of 12..18 qubits: 8.1 -> 5.3 ms.
 // An autotuner times (workgroup size, LDS tile) candidates and keeps the
 // fastest.
 //
@@ -40,7 +47,16 @@ struct Desc {
     uint32_t phase_begin, phase_count;
     int32_t n;
     int32_t index;  // position in the caller's order
+    uint32_t part_begin;  // first of its tiles' <sum Z> partials
+    uint32_t pad;
 };
+
+// What one workgroup does: phase `phase` of tile `tile` of state `desc`; the
+// tile's <sum Z> goes to `part` unless that is kNoPart.
+struct BatchItem {
+    uint32_t desc, tile, phase, part;
+};
+constexpr uint32_t kNoPart = ~0u;
 
 __device__ __forceinline__ uint32_t ins0(uint32_t p, int t) { return ((p >> t) << (t + 1)) | (p & ((1u << t) - 1u)); }
 
@@ -382,73 +398,101 @@ __device__ double block_sum(double acc, double* s_red) {
     return s;
 }
 
-// Persistent: each workgroup takes states from the queue until none is left.
-// A state of n qubits is swept in tiles of 2^min(n, lds_qubits) amplitudes;
-// its first phase starts from |0..0> in LDS, its last phase reduces
+// One item per workgroup.  A state of n qubits is swept in tiles of
+// 2^min(n, lds_qubits) amplitudes; its first phase starts from |0..0> in LDS
+// (where every tile but the first stays zero), its last phase reduces
 // <sum Z> while storing.
 template <int BLOCK>
-__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void k_batch(const Desc* __restrict__ desc, int count,
-                                                  const BatchPhase* __restrict__ phases,
-                                                  const BatchSeg* __restrict__ segs, const BatchOp* __restrict__ ops,
-                                                  float2* __restrict__ pool, double* __restrict__ out,
-                                                  unsigned* __restrict__ queue, int lds_qubits) {
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void k_batch(
+    const Desc* __restrict__ desc, const BatchItem* __restrict__ items, const BatchPhase* __restrict__ phases,
+    const BatchSeg* __restrict__ segs, const BatchOp* __restrict__ ops, float2* __restrict__ pool,
+    double* __restrict__ part, int lds_qubits) {
     extern __shared__ float2 lds[];
-    __shared__ int s_idx;
     __shared__ double s_red[BLOCK / 64];
     const int tid = threadIdx.x;
-    while (true) {
-        if (tid == 0) s_idx = (int)atomicAdd(queue, 1u);
-        __syncthreads();
-        const int k = __builtin_amdgcn_readfirstlane(s_idx);
-        __syncthreads();
-        if (k >= count) break;  // every wave of the workgroup leaves together
-        const Desc d = desc[k];
-        float2* hbm = pool + d.amp_offset;
-        const int m = d.n < lds_qubits ? d.n : lds_qubits;
-        const uint32_t T = 1u << m, tiles = 1u << (d.n - m);
-        double acc = 0.0;
-        for (uint32_t p = 0; p < d.phase_count; ++p) {
-            const BatchPhase ph = phases[d.phase_begin + p];
-            const bool last = p + 1 == d.phase_count;
-            for (uint32_t t = 0; t < tiles; ++t) {
-                const uint32_t g = deposit(t, ph.gbits);
-                if (p == 0) {
-                    for (uint32_t j = tid; j < T; j += BLOCK)
-                        lds[lds_slot(j)] = make_float2(t == 0 && j == 0 ? 1.f : 0.f, 0.f);
-                } else {
-                    for (uint32_t j = tid; j < T; j += BLOCK) lds[lds_slot(j)] = hbm[spread(j, ph.gbits) | g];
-                }
-                __syncthreads();
-                for (uint32_t s = 0; s < ph.seg_count; ++s) {
-                    const BatchSeg sg = segs[ph.seg_begin + s];
-                    if (sg.rmask) {
-                        run_reg_segment<BLOCK>(lds, T, sg, ops, g);
-                        continue;
-                    }
-                    for (uint32_t o = 0; o < sg.op_count; ++o) {
-                        BatchOp e = ops[sg.op_begin + o];
-                        if (!resolve(e, g)) continue;  // uniform over the workgroup
-                        apply_block<BLOCK>(lds, T, e);
-                        __syncthreads();
-                    }
-                }
-                for (uint32_t j = tid; j < T; j += BLOCK) {
-                    const float2 v = lds[lds_slot(j)];
-                    const uint32_t i = spread(j, ph.gbits) | g;
-                    if (last) acc += ((double)v.x * v.x + (double)v.y * v.y) * (double)(d.n - 2 * (int)__popc(i));
-                    hbm[i] = v;
-                }
-                __syncthreads();  // the next tile's load reuses the LDS
-            }
+    const BatchItem it = items[blockIdx.x];
+    const Desc d = desc[it.desc];
+    float2* hbm = pool + d.amp_offset;
+    const int m = d.n < lds_qubits ? d.n : lds_qubits;
+    const uint32_t T = 1u << m;
+    const BatchPhase ph = phases[d.phase_begin + it.phase];
+    const uint32_t g = deposit(it.tile, ph.gbits);
+    if (it.phase == 0) {
+        for (uint32_t j = tid; j < T; j += BLOCK)
+            lds[lds_slot(j)] = make_float2(it.tile == 0 && j == 0 ? 1.f : 0.f, 0.f);
+    } else {
+        for (uint32_t j = tid; j < T; j += BLOCK) lds[lds_slot(j)] = hbm[spread(j, ph.gbits) | g];
+    }
+    __syncthreads();
+    const uint32_t seg_count = it.phase == 0 && it.tile != 0 ? 0u : ph.seg_count;
+    for (uint32_t s = 0; s < seg_count; ++s) {
+        const BatchSeg sg = segs[ph.seg_begin + s];
+        if (sg.rmask) {
+            run_reg_segment<BLOCK>(lds, T, sg, ops, g);
+            continue;
         }
+        for (uint32_t o = 0; o < sg.op_count; ++o) {
+            BatchOp e = ops[sg.op_begin + o];
+            if (!resolve(e, g)) continue;  // uniform over the workgroup
+            apply_block<BLOCK>(lds, T, e);
+            __syncthreads();
+        }
+    }
+    double acc = 0.0;
+    for (uint32_t j = tid; j < T; j += BLOCK) {
+        const float2 v = lds[lds_slot(j)];
+        const uint32_t i = spread(j, ph.gbits) | g;
+        if (it.part != kNoPart) acc += ((double)v.x * v.x + (double)v.y * v.y) * (double)(d.n - 2 * (int)__popc(i));
+        hbm[i] = v;
+    }
+    if (it.part != kNoPart) {
         const double s = block_sum<BLOCK>(acc, s_red);
-        if (tid == 0) out[d.index] = s;
-        __syncthreads();
+        if (tid == 0) part[it.part] = s;
     }
 }
 
-__global__ void k_reset_queue(unsigned* q) {
-    if (threadIdx.x == 0 && blockIdx.x == 0) *q = 0u;
+// <sum Z> of each state: its tiles' partials in order.
+__global__ __launch_bounds__(64) void k_batch_expect(const Desc* __restrict__ desc, int count,
+                                                     const double* __restrict__ part, int lds_qubits,
+                                                     double* __restrict__ out) {
+    const int k = blockIdx.x * 64 + threadIdx.x;
+    if (k >= count) return;
+    const Desc d = desc[k];
+    const uint32_t tiles = d.n > lds_qubits ? 1u << (d.n - lds_qubits) : 1u;
+    double s = 0.0;
+    for (uint32_t t = 0; t < tiles; ++t) s += part[d.part_begin + t];
+    out[d.index] = s;
+}
+
+// The items of all levels (level p: the p-th phase of every state that has
+// one, in the order of `desc`), and where each level begins.  Sets the
+// states' part_begin; `parts` = number of partials (0: no <sum Z> wanted).
+struct Levels {
+    std::vector<BatchItem> items;
+    std::vector<uint32_t> begin;  // levels + 1
+    uint32_t parts = 0;
+};
+
+Levels make_levels(std::vector<Desc>& desc, int lds_qubits, bool expect) {
+    Levels l;
+    auto tiles = [&](const Desc& d) { return d.n > lds_qubits ? 1u << (d.n - lds_qubits) : 1u; };
+    uint32_t levels = 0;
+    for (Desc& d : desc) {
+        d.part_begin = l.parts;
+        if (expect) l.parts += tiles(d);
+        levels = std::max(levels, d.phase_count);
+    }
+    for (uint32_t p = 0; p < levels; ++p) {
+        l.begin.push_back((uint32_t)l.items.size());
+        for (uint32_t k = 0; k < desc.size(); ++k) {
+            if (p >= desc[k].phase_count) continue;
+            const bool last = p + 1 == desc[k].phase_count;
+            for (uint32_t t = 0; t < tiles(desc[k]); ++t)
+                l.items.push_back({k, t, p, expect && last ? desc[k].part_begin + t : kNoPart});
+        }
+    }
+    l.begin.push_back((uint32_t)l.items.size());
+    return l;
 }
 
 using cd = std::complex<double>;
@@ -762,7 +806,10 @@ struct aqs_batch_s {
         std::vector<BatchOp> ops;
         std::vector<BatchSeg> segs;
         std::vector<BatchPhase> phases;
+        Levels levels;
         void* d_desc = nullptr;
+        void* d_items = nullptr;
+        void* d_part = nullptr;
         void* d_ops = nullptr;
         void* d_segs = nullptr;
         void* d_phases = nullptr;
@@ -777,7 +824,6 @@ struct aqs_batch_s {
     size_t source_ops = 0;
     float2* d_pool = nullptr;
     double* d_out = nullptr;
-    unsigned* d_queue = nullptr;
     hipStream_t stream = nullptr;
     int block = 512;
     int lds_qubits = 13;
@@ -793,10 +839,12 @@ namespace {
 
 void free_prog(aqs_batch_s::Prog& p) {
     if (p.d_desc) (void)hipFree(p.d_desc);
+    if (p.d_items) (void)hipFree(p.d_items);
+    if (p.d_part) (void)hipFree(p.d_part);
     if (p.d_ops) (void)hipFree(p.d_ops);
     if (p.d_segs) (void)hipFree(p.d_segs);
     if (p.d_phases) (void)hipFree(p.d_phases);
-    p.d_desc = p.d_ops = p.d_segs = p.d_phases = nullptr;
+    p.d_desc = p.d_items = p.d_part = p.d_ops = p.d_segs = p.d_phases = nullptr;
 }
 
 // The program for LDS tiles of 2^m amplitudes, built and uploaded on first use.
@@ -818,11 +866,16 @@ aqs_batch_s::Prog& prog_for(aqs_batch b, int m) {
         }
         if (p.ops.size() >= (1ull << 32) || p.segs.size() >= (1ull << 32))
             fail(AQS_ERR_INVALID_ARGUMENT, "batch program exceeds 2^32 ops");
+        p.levels = make_levels(p.desc, m, true);
         AQS_HIP(hipMalloc(&p.d_desc, sizeof(Desc) * p.desc.size()));
+        AQS_HIP(hipMalloc(&p.d_items, sizeof(BatchItem) * p.levels.items.size()));
+        AQS_HIP(hipMalloc(&p.d_part, sizeof(double) * p.levels.parts));
         AQS_HIP(hipMalloc(&p.d_ops, sizeof(BatchOp) * std::max<size_t>(1, p.ops.size())));
         AQS_HIP(hipMalloc(&p.d_segs, sizeof(BatchSeg) * std::max<size_t>(1, p.segs.size())));
         AQS_HIP(hipMalloc(&p.d_phases, sizeof(BatchPhase) * p.phases.size()));
         AQS_HIP(hipMemcpy(p.d_desc, p.desc.data(), sizeof(Desc) * p.desc.size(), hipMemcpyHostToDevice));
+        AQS_HIP(hipMemcpy(p.d_items, p.levels.items.data(), sizeof(BatchItem) * p.levels.items.size(),
+                          hipMemcpyHostToDevice));
         if (!p.ops.empty())
             AQS_HIP(hipMemcpy(p.d_ops, p.ops.data(), sizeof(BatchOp) * p.ops.size(), hipMemcpyHostToDevice));
         if (!p.segs.empty())
@@ -850,42 +903,44 @@ size_t lds_bytes_for(int lds_qubits) {
     return sizeof(float2) * (T + (T >> 5));
 }
 
-void launch_kernel(aqs_batch b, int block, int lds_qubits, int grid) {
-    aqs_batch_s::Prog& p = prog_for(b, lds_qubits);
+// The launches of all levels.
+void launch_levels(const Desc* desc, const BatchItem* items, const std::vector<uint32_t>& begin,
+                   const BatchPhase* phases, const BatchSeg* segs, const BatchOp* ops, float2* pool, double* part,
+                   int block, int lds_qubits, hipStream_t stream) {
     const size_t lds_bytes = lds_bytes_for(lds_qubits);
-    const auto* desc = (const Desc*)p.d_desc;
-    const auto* phases = (const BatchPhase*)p.d_phases;
-    const auto* segs = (const BatchSeg*)p.d_segs;
-    const auto* ops = (const BatchOp*)p.d_ops;
-    hipLaunchKernelGGL(k_reset_queue, dim3(1), dim3(64), 0, b->stream, b->d_queue);
-    switch (block) {
-        case 256:
-            hipLaunchKernelGGL(k_batch<256>, dim3(grid), dim3(256), lds_bytes, b->stream, desc, b->count, phases, segs, ops,
-                               b->d_pool, b->d_out, b->d_queue, lds_qubits);
-            break;
-        case 512:
-            hipLaunchKernelGGL(k_batch<512>, dim3(grid), dim3(512), lds_bytes, b->stream, desc, b->count, phases, segs, ops,
-                               b->d_pool, b->d_out, b->d_queue, lds_qubits);
-            break;
-        default:
-            hipLaunchKernelGGL(k_batch<1024>, dim3(grid), dim3(1024), lds_bytes, b->stream, desc, b->count, phases, segs, ops,
-                               b->d_pool, b->d_out, b->d_queue, lds_qubits);
-            break;
+    for (size_t p = 0; p + 1 < begin.size(); ++p) {
+        const dim3 grid(begin[p + 1] - begin[p]);
+        const BatchItem* it = items + begin[p];
+        switch (block) {
+            case 256:
+                hipLaunchKernelGGL(k_batch<256>, grid, dim3(256), lds_bytes, stream, desc, it, phases, segs, ops, pool,
+                                   part, lds_qubits);
+                break;
+            case 512:
+                hipLaunchKernelGGL(k_batch<512>, grid, dim3(512), lds_bytes, stream, desc, it, phases, segs, ops, pool,
+                                   part, lds_qubits);
+                break;
+            default:
+                hipLaunchKernelGGL(k_batch<1024>, grid, dim3(1024), lds_bytes, stream, desc, it, phases, segs, ops,
+                                   pool, part, lds_qubits);
+                break;
+        }
     }
     AQS_HIP(hipGetLastError());
 }
 
-int grid_for(int block, int lds_qubits) {
-    int dev = current_device();
-    hipDeviceProp_t prop;
-    AQS_HIP(hipGetDeviceProperties(&prop, dev));
-    const size_t lds_bytes = lds_bytes_for(lds_qubits);
-    const size_t lds_per_cu = 160 * 1024;
-    int per_cu_lds = (int)std::max<size_t>(1, lds_per_cu / (lds_bytes + 1024));
-    int per_cu_threads = std::max(1, 2048 / block);
-    int per_cu = std::min(per_cu_lds, per_cu_threads);
-    return prop.multiProcessorCount * per_cu;
+void launch_kernel(aqs_batch b, int block, int lds_qubits) {
+    aqs_batch_s::Prog& p = prog_for(b, lds_qubits);
+    launch_levels((const Desc*)p.d_desc, (const BatchItem*)p.d_items, p.levels.begin, (const BatchPhase*)p.d_phases,
+                  (const BatchSeg*)p.d_segs, (const BatchOp*)p.d_ops, b->d_pool, (double*)p.d_part, block, lds_qubits,
+                  b->stream);
+    hipLaunchKernelGGL(k_batch_expect, dim3((b->count + 63) / 64), dim3(64), 0, b->stream, (const Desc*)p.d_desc,
+                       b->count, (const double*)p.d_part, lds_qubits, b->d_out);
+    AQS_HIP(hipGetLastError());
 }
+
+// Workgroups of the first level.
+int first_grid(aqs_batch b) { return (int)prog_for(b, b->lds_qubits).levels.begin[1]; }
 
 void set_lds_limit() {
     const int bytes = 160 * 1024 - 4096;
@@ -899,7 +954,7 @@ void build_graph(aqs_batch b) {
     prog_for(b, b->lds_qubits);  // allocates and uploads: not allowed while capturing
     AQS_HIP(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
     try {
-        launch_kernel(b, b->block, b->lds_qubits, b->grid);
+        launch_kernel(b, b->block, b->lds_qubits);
     } catch (...) {
         hipGraph_t g;
         (void)hipStreamEndCapture(b->stream, &g);
@@ -916,7 +971,7 @@ void build_graph(aqs_batch b) {
 double time_config(aqs_batch b, int block, int lds_qubits) {
     b->block = block;
     b->lds_qubits = lds_qubits;
-    b->grid = grid_for(block, lds_qubits);
+    b->grid = first_grid(b);
     build_graph(b);
     AQS_HIP(hipGraphLaunch(b->exec, b->stream));
     float t[3];
@@ -945,7 +1000,7 @@ namespace aqs_hip {
 namespace {
 
 constexpr size_t kArenaAlign = 256;
-constexpr int kGroupRegions = 10;  // aligned regions of the arena layout
+constexpr int kGroupRegions = 9;  // aligned regions of the arena layout
 
 size_t align_up(size_t x) { return (x + kArenaAlign - 1) / kArenaAlign * kArenaAlign; }
 
@@ -953,18 +1008,20 @@ size_t align_up(size_t x) { return (x + kArenaAlign - 1) / kArenaAlign * kArenaA
 
 // A member's program holds at most nops absorbed ops, each cut into at most
 // three (a swap becomes three X gates), at most one segment per op and at
-// most one phase per absorbed op plus one.
+// most one phase per absorbed op plus one, each phase one item per tile.
 size_t group_item_bytes(int n, size_t nops, uint32_t shots) {
-    const size_t prog = sizeof(Desc) + (nops + 1) * sizeof(BatchPhase) + 3 * nops * sizeof(BatchSeg) +
-                        3 * nops * sizeof(BatchOp);
-    const size_t io = sizeof(double) * 2 + 2 * sizeof(uint64_t) * (size_t)shots;  // expectation, norm, u, indices
+    const size_t tiles = n > kGroupLdsQubits ? (size_t)1 << (n - kGroupLdsQubits) : 1;
+    const size_t items = n > kGroupLdsQubits ? (nops + 1) * tiles : 1;
+    const size_t prog = sizeof(Desc) + items * sizeof(BatchItem) + (nops + 1) * sizeof(BatchPhase) +
+                        3 * nops * sizeof(BatchSeg) + 3 * nops * sizeof(BatchOp);
+    const size_t io = sizeof(double) + 2 * sizeof(uint64_t) * (size_t)shots;  // norm, u, indices
     return prog + io + align_up(sizeof(float2) << n) + align_up(sample_norm_scratch_bytes(n)) +
            kGroupRegions * kArenaAlign;
 }
 
 void run_group(GroupItem* items, int count, void* arena, size_t arena_bytes, hipStream_t stream) {
     if (count < 1) return;
-    // programs, biggest state first (the persistent grid takes states in order)
+    // programs, biggest state first (workgroups start in item order)
     std::vector<int> order(count);
     std::vector<uint64_t> cost(count);
     std::vector<std::vector<BatchOp>> flat(count);
@@ -986,8 +1043,8 @@ void run_group(GroupItem* items, int count, void* arena, size_t arena_bytes, hip
         shot_off[k] = shots_total;
         shots_total += items[k].shots;
     }
-    // arena layout: queue | <sum Z> | upload (desc, phases, segs, ops, u) |
-    // download (norms, indices) | states | sampling scratch
+    // arena layout: upload (desc, items, phases, segs, ops, u) | download
+    // (norms, indices) | states | sampling scratch
     size_t off = 0;
     auto take = [&](size_t bytes) {
         const size_t at = off;
@@ -1004,9 +1061,9 @@ void run_group(GroupItem* items, int count, void* arena, size_t arena_bytes, hip
         items[k].passes = d.phase_count;
         desc.push_back(d);
     }
-    const size_t o_queue = take(sizeof(unsigned));
-    const size_t o_zout = take(sizeof(double) * count);
+    const Levels levels = make_levels(desc, kGroupLdsQubits, false);
     const size_t o_desc = take(sizeof(Desc) * desc.size());
+    const size_t o_items = take(sizeof(BatchItem) * levels.items.size());
     const size_t o_phases = take(sizeof(BatchPhase) * phases.size());
     const size_t o_segs = take(sizeof(BatchSeg) * std::max<size_t>(1, segs.size()));
     const size_t o_ops = take(sizeof(BatchOp) * std::max<size_t>(1, ops.size()));
@@ -1024,6 +1081,7 @@ void run_group(GroupItem* items, int count, void* arena, size_t arena_bytes, hip
     // one upload: desc .. u are contiguous
     std::vector<char> up(o_norm - o_desc);
     std::memcpy(up.data(), desc.data(), sizeof(Desc) * desc.size());
+    std::memcpy(up.data() + (o_items - o_desc), levels.items.data(), sizeof(BatchItem) * levels.items.size());
     std::memcpy(up.data() + (o_phases - o_desc), phases.data(), sizeof(BatchPhase) * phases.size());
     if (!segs.empty()) std::memcpy(up.data() + (o_segs - o_desc), segs.data(), sizeof(BatchSeg) * segs.size());
     if (!ops.empty()) std::memcpy(up.data() + (o_ops - o_desc), ops.data(), sizeof(BatchOp) * ops.size());
@@ -1034,14 +1092,10 @@ void run_group(GroupItem* items, int count, void* arena, size_t arena_bytes, hip
     AQS_HIP(hipMemcpyAsync(base + o_desc, up.data(), up.size(), hipMemcpyHostToDevice, stream));
 
     set_lds_limit();
-    hipLaunchKernelGGL(k_reset_queue, dim3(1), dim3(64), 0, stream, (unsigned*)(base + o_queue));
-    const unsigned grid = (unsigned)std::min(grid_for(kGroupBlock, kGroupLdsQubits), count);
-    hipLaunchKernelGGL(k_batch<kGroupBlock>, dim3(grid), dim3(kGroupBlock), lds_bytes_for(kGroupLdsQubits), stream,
-                       (const Desc*)(base + o_desc), count, (const BatchPhase*)(base + o_phases),
-                       (const BatchSeg*)(base + o_segs), (const BatchOp*)(base + o_ops),
-                       (float2*)(base + o_state[0]), (double*)(base + o_zout), (unsigned*)(base + o_queue),
-                       kGroupLdsQubits);
-    AQS_HIP(hipGetLastError());
+    launch_levels((const Desc*)(base + o_desc), (const BatchItem*)(base + o_items), levels.begin,
+                  (const BatchPhase*)(base + o_phases), (const BatchSeg*)(base + o_segs),
+                  (const BatchOp*)(base + o_ops), (float2*)(base + o_state[0]), nullptr, kGroupBlock, kGroupLdsQubits,
+                  stream);
     for (int k = 0; k < count; ++k)
         queue_sample_norm(base + o_state[k], items[k].n, base + o_scr[k],
                           (const double*)(base + o_u) + shot_off[k], items[k].shots,
@@ -1100,10 +1154,9 @@ aqs_status aqs_batch_create(int count, const int* nqubits, const aqs_op* ops, co
             AQS_HIP(hipEventCreate(&b->e1));
             AQS_HIP(hipMalloc(&b->d_pool, sizeof(float2) * amps));
             AQS_HIP(hipMalloc(&b->d_out, sizeof(double) * count));
-            AQS_HIP(hipMalloc(&b->d_queue, 256));
             set_lds_limit();
             prog_for(b, b->lds_qubits);
-            b->grid = grid_for(b->block, b->lds_qubits);
+            b->grid = first_grid(b);
         } catch (...) {
             aqs_batch_destroy(b);
             throw;
@@ -1128,7 +1181,7 @@ aqs_status aqs_batch_autotune(aqs_batch b, int* block, int* lds_qubits, double* 
             }
         b->block = bb;
         b->lds_qubits = bl;
-        b->grid = grid_for(bb, bl);
+        b->grid = first_grid(b);
         b->tuned = true;
         destroy_graph(b);
         for (auto it = b->progs.begin(); it != b->progs.end();) {
@@ -1154,7 +1207,7 @@ aqs_status aqs_batch_configure(aqs_batch b, int block, int lds_qubits) {
         prog_for(b, lds_qubits);
         b->block = block;
         b->lds_qubits = lds_qubits;
-        b->grid = grid_for(block, lds_qubits);
+        b->grid = first_grid(b);
         destroy_graph(b);
     });
 }
@@ -1207,7 +1260,6 @@ aqs_status aqs_batch_destroy(aqs_batch b) {
         for (auto& kv : b->progs) free_prog(kv.second);
         if (b->d_pool) (void)hipFree(b->d_pool);
         if (b->d_out) (void)hipFree(b->d_out);
-        if (b->d_queue) (void)hipFree(b->d_queue);
         if (b->e0) (void)hipEventDestroy(b->e0);
         if (b->e1) (void)hipEventDestroy(b->e1);
         if (b->stream) (void)hipStreamDestroy(b->stream);

@@ -30,9 +30,13 @@ ARCH = "gfx950"
 # -fcx-limited-range: host complex products by the textbook formula (every
 # operand is a gate or unitary entry, |x| <= 1) instead of a library call
 # that rescues overflow and NaN.
+# -structurizecfg-skip-uniform-regions: the op switches of the tile, batch and
+# run kernels branch on scalars; without it they become chains of
+# flag-and-branch joins that every op walks through.
 HIP_FLAGS = [
     f"--offload-arch={ARCH}", "-O3", "-fPIC", "-std=c++17", "-Wall", "-fcx-limited-range",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+    "-mllvm", "-structurizecfg-skip-uniform-regions=true",
     "-I", INCLUDE, "-I", CSRC,
 ]
 

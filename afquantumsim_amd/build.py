@@ -41,7 +41,7 @@ HIP_FLAGS = [
 ]
 
 HIP_SOURCES = ["state.hip", "gates.hip", "mfma.hip", "diag.hip", "perm.hip", "tile.hip", "measure.hip", "batch.hip",
-               "fusion.cpp", "tiling.cpp", "serve_core.cpp", "serve.cpp"]
+               "runs.hip", "runs.cpp", "fusion.cpp", "tiling.cpp", "serve_core.cpp", "serve.cpp"]
 CPP_SOURCES = ["quantum.cpp", "quantum_algo.cpp", "quantum_gates.cpp"]  # algo_bench.cpp is a program
 
 

@@ -25,8 +25,8 @@ std::mt19937 g_rd_gen{g_dv()};
 std::uniform_real_distribution<float> g_lin_dist{0.0f, 1.0f};
 
 std::unordered_map<std::string, std::shared_ptr<QCircuit>> g_cached_circuits;
-// States up to this size run op sequences in LDS-resident batches (aqs_apply
-// on a complex64 state); simulate() and compile() hand them whole runs.
+// States up to this size are one LDS-resident tile for aqs_apply, which runs
+// their op sequences faster than fused passes: compile() keeps the ops.
 constexpr uint32_t kSmallStateQubits = 12;
 
 void check(aqs_status st) {
@@ -480,17 +480,8 @@ void QSimulator::simulate(const QCircuit& circuit) {
     circuit.run_compiled(statevector_.handle());
     QCircuit temp{qubit_count()};
     detail::Sink sink;
-    if (qubit_count() > kSmallStateQubits) {
-        // one aqs_apply per op, as the gates emit them
-        sink.state = statevector_.handle();
-        temp.sink_ = &sink;
-        for (size_t i = circuit.cached_index_; i < circuit.gate_list().size(); ++i)
-            circuit.gate_list()[i]->operator()(temp);
-        temp.sink_ = nullptr;
-        return;
-    }
-    // Small states: the ops are collected and applied by one aqs_apply, which
-    // runs them in LDS-resident batches instead of one launch each.
+    // The ops are collected and applied by one aqs_apply, which runs them in
+    // LDS-resident tiles instead of one launch each.
     std::vector<detail::OpRecord> rec;
     sink.record = &rec;
     temp.sink_ = &sink;

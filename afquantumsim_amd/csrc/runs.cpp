@@ -1,0 +1,461 @@
+// Planner of runs of uncompiled ops (runs.h).
+#include "runs.h"
+
+#include <algorithm>
+#include <complex>
+#include <cstring>
+
+#include "rotation.h"
+
+using namespace aqs_hip;
+
+namespace {
+
+using cd = std::complex<double>;
+
+enum Kind : uint8_t { K_MATP, K_REAL, K_MAT, K_X, K_PHASE };
+
+struct POp {
+    Kind kind;
+    uint8_t t = 0;               // target bit (K_PHASE: unused)
+    uint32_t nd = 0, dg = 0;     // index bits changed, index bits read or multiplied on
+    uint32_t all = 0, any = 0;   // controls (K_PHASE: `all` = required bits)
+    double m[8] = {};
+};
+
+struct M2 {
+    cd a[4];
+};
+
+class Planner {
+   public:
+    Planner(int n, int m, int precision) : n_(n), m_(m), R_(precision == AQS_C64 ? 1u : 2u), pend_(n), has_(n, 0) {}
+
+    std::vector<RunLaunch> run(const aqs_op* ops, size_t count) {
+        list_.reserve(count + (size_t)n_);
+        for (size_t i = 0; i < count; ++i) absorb(ops[i]);
+        for (int b = 0; b < n_; ++b) flush(b);
+        rem_.resize(list_.size());
+        for (uint32_t i = 0; i < rem_.size(); ++i) rem_[i] = i;
+        while (!rem_.empty()) pass();
+        return std::move(out_);
+    }
+
+   private:
+    int n_, m_;
+    uint32_t R_;
+    std::vector<M2> pend_;   // per index bit: one-qubit gates not yet emitted
+    std::vector<char> has_;
+    std::vector<POp> list_;
+    std::vector<uint32_t> rem_, next_, members_, left_;
+    std::vector<RunLaunch> out_;
+
+    // ---- lowering -----------------------------------------------------------
+
+    uint32_t bit(int q) const { return 1u << (n_ - 1 - q); }
+
+    void push_phase(uint32_t mask, cd z) {
+        if (z == cd(1)) return;
+        POp o{K_PHASE};
+        o.dg = o.all = mask;
+        o.m[0] = z.real();
+        o.m[1] = z.imag();
+        list_.push_back(o);
+    }
+
+    void push_pair(Kind k, int t, uint32_t all, uint32_t any, const double* m, int nm) {
+        POp o{k};
+        o.t = (uint8_t)t;
+        o.nd = 1u << t;
+        o.all = all;
+        o.any = any;
+        o.dg = all | any;
+        for (int i = 0; i < nm; ++i) o.m[i] = m[i];
+        list_.push_back(o);
+    }
+
+    // A 2x2 on bit t under controls: real matrices (H, RotY) as real ones.
+    void push_mat(int t, uint32_t all, uint32_t any, const M2& u) {
+        bool real = !any;
+        for (const cd& x : u.a) real = real && x.imag() == 0.0;
+        if (real) {
+            const double m[4] = {u.a[0].real(), u.a[1].real(), u.a[2].real(), u.a[3].real()};
+            push_pair(K_REAL, t, all, any, m, 4);
+        } else {
+            double m[8];
+            for (int i = 0; i < 4; ++i) {
+                m[2 * i] = u.a[i].real();
+                m[2 * i + 1] = u.a[i].imag();
+            }
+            push_pair(K_MAT, t, all, any, m, 8);
+        }
+    }
+
+    void push_diag(int t, uint32_t all, cd d0, cd d1) {
+        push_phase(all, d0);
+        push_phase(all | (1u << t), d1 / d0);
+    }
+
+    // Emits bit b's pending 2x2, before a gate that changes the bit.
+    void flush(int b) {
+        if (!has_[b]) return;
+        has_[b] = 0;
+        const M2& u = pend_[b];
+        if (u.a[1] == cd(0) && u.a[2] == cd(0) && u.a[0] != cd(0))
+            push_diag(b, 0, u.a[0], u.a[3]);
+        else if (u.a[0] == cd(0) && u.a[3] == cd(0) && u.a[1] == cd(1) && u.a[2] == cd(1))
+            push_pair(K_X, b, 0, 0, nullptr, 0);
+        else
+            push_mat(b, 0, 0, u);
+    }
+
+    // Before a gate that uses the bit only diagonally: the non-diagonal part
+    // is emitted, a diagonal on its left stays pending (it commutes with that
+    // gate).  U = diag(g0, g1) R diag(1, z) takes 10 multiply-adds per pair
+    // as a rotation after a phase, 16 as a 2x2.
+    void flush_rotation(int b) {
+        if (!has_[b]) return;
+        M2& u = pend_[b];
+        if (u.a[1] == cd(0) && u.a[2] == cd(0)) return;
+        if (u.a[0] == cd(0) && u.a[3] == cd(0)) {  // diag(u01, u10) X
+            push_pair(K_X, b, 0, 0, nullptr, 0);
+            u.a[0] = u.a[1];
+            u.a[3] = u.a[2];
+            u.a[1] = u.a[2] = 0;
+            if (u.a[0] == cd(1) && u.a[3] == cd(1)) has_[b] = 0;
+            return;
+        }
+        bool real = true;
+        for (const cd& x : u.a) real = real && x.imag() == 0.0;
+        RotationForm f;
+        // complex128 states, the FP64 reference, keep the matrix as it was
+        // given (the form holds to 1e-12, and shears round more often)
+        if (real || R_ == 2 || !factor_rotation(u.a[0], u.a[1], u.a[2], u.a[3], f)) {
+            flush(b);
+            return;
+        }
+        double t, su, nr;
+        rotation_shears(f.c, f.s, t, su, nr);
+        const double m[4] = {t, su, f.z.real(), f.z.imag()};
+        push_pair(K_MATP, b, 0, 0, m, 4);
+        u.a[0] = f.g0 * nr;
+        u.a[1] = u.a[2] = 0;
+        u.a[3] = f.g1 * nr;
+    }
+
+    void flush_rotations(uint32_t mask) {
+        for (; mask; mask &= mask - 1u) flush_rotation(__builtin_ctz(mask));
+    }
+
+    void absorb_1q(int b, const M2& u) {
+        if (!has_[b]) {
+            pend_[b] = u;
+            has_[b] = 1;
+            return;
+        }
+        const M2 p = pend_[b];
+        M2& r = pend_[b];
+        r.a[0] = u.a[0] * p.a[0] + u.a[1] * p.a[2];
+        r.a[1] = u.a[0] * p.a[1] + u.a[1] * p.a[3];
+        r.a[2] = u.a[2] * p.a[0] + u.a[3] * p.a[2];
+        r.a[3] = u.a[2] * p.a[1] + u.a[3] * p.a[3];
+    }
+
+    void absorb(const aqs_op& op) {
+        uint32_t ctrl = 0, more = 0;
+        for (int j = 0; j < op.ncontrols; ++j) ctrl |= bit(op.controls[j]);
+        for (uint64_t x = op.more_controls; x; x &= x - 1) more |= bit(__builtin_ctzll(x));
+        // PHASE takes its controls as required bits whatever the flag
+        const bool any = (op.flags & AQS_CTRL_ANY) && ctrl && op.kind != AQS_OP_PHASE;
+        const uint32_t all = (any ? 0u : ctrl) | more, anym = any ? ctrl : 0u;
+        const int t = n_ - 1 - op.targets[0];
+        M2 u{};
+        switch (op.kind) {
+            case AQS_OP_MAT1:
+                for (int i = 0; i < 4; ++i) u.a[i] = cd(op.m[2 * i], op.m[2 * i + 1]);
+                break;
+            case AQS_OP_DIAG1:
+                u.a[0] = cd(op.m[0], op.m[1]);
+                u.a[3] = cd(op.m[6], op.m[7]);
+                break;
+            case AQS_OP_X:
+                u.a[1] = u.a[2] = 1;
+                break;
+            default:
+                break;
+        }
+        switch (op.kind) {
+            case AQS_OP_MAT1:
+            case AQS_OP_DIAG1:
+            case AQS_OP_X:
+                if (!(all | anym)) {
+                    absorb_1q(t, u);
+                    return;
+                }
+                flush_rotations(all | anym);
+                if (op.kind == AQS_OP_DIAG1 && !any && u.a[0] != cd(0)) {
+                    flush_rotation(t);
+                    push_diag(t, all, u.a[0], u.a[3]);
+                    return;
+                }
+                flush(t);
+                if (op.kind == AQS_OP_X)
+                    push_pair(K_X, t, all, anym, nullptr, 0);
+                else
+                    push_mat(t, all, anym, u);
+                return;
+            case AQS_OP_PHASE: {
+                uint32_t mask = all;
+                for (int j = 0; j < op.ntargets; ++j) mask |= bit(op.targets[j]);
+                const cd z(op.m[0], op.m[1]);
+                if (!(mask & (mask - 1u))) {
+                    u.a[0] = 1;
+                    u.a[3] = z;
+                    absorb_1q(__builtin_ctz(mask), u);
+                    return;
+                }
+                flush_rotations(mask);
+                push_phase(mask, z);
+                return;
+            }
+            default: {  // SWAP: CX(a -> b), X on a where b and the controls hold, CX(a -> b)
+                const int a = t, b = n_ - 1 - op.targets[1];
+                flush_rotations(all | anym);
+                flush(a);
+                flush(b);
+                push_pair(K_X, b, 1u << a, 0, nullptr, 0);
+                push_pair(K_X, a, all | (1u << b), anym, nullptr, 0);
+                push_pair(K_X, b, 1u << a, 0, nullptr, 0);
+                return;
+            }
+        }
+    }
+
+    // ---- passes and segments ------------------------------------------------
+
+    struct Passed {  // index bits that the ops passed over change / use diagonally
+        uint32_t nd = 0, dg = 0;
+        bool blocks(const POp& o) const { return (o.nd & (nd | dg)) || (o.dg & nd); }
+        void over(const POp& o) {
+            nd |= o.nd;
+            dg |= o.dg;
+        }
+    };
+
+    void pass() {
+        const uint32_t all = (1u << n_) - 1u;
+        uint32_t local = (1u << std::min(5, m_)) - 1u;
+        Passed st;
+        members_.clear();
+        next_.clear();
+        size_t i = 0;
+        for (; i < rem_.size() && st.nd != all; ++i) {
+            const POp& o = list_[rem_[i]];
+            if (!st.blocks(o) && __builtin_popcount(local | o.nd) <= m_) {
+                local |= o.nd;
+                members_.push_back(rem_[i]);
+            } else {
+                st.over(o);
+                next_.push_back(rem_[i]);
+            }
+        }
+        next_.insert(next_.end(), rem_.begin() + (long)i, rem_.end());
+        rem_.swap(next_);
+        for (int b = 0; __builtin_popcount(local) < m_; ++b) local |= 1u << b;
+        segments(local);
+    }
+
+    static uint32_t compress(uint32_t mask, uint32_t local) {
+        uint32_t r = 0, k = 0;
+        for (uint32_t l = local; l; l &= l - 1u, ++k)
+            if (mask & l & (0u - l)) r |= 1u << k;
+        return r;
+    }
+
+    // The launch being written.
+    uint32_t local_ = 0, rmask_ = 0;  // tile bits; register bits (index bits)
+    uint32_t seg_at_ = 0, ops_ = 0;
+
+    std::vector<uint32_t>& words() { return out_.back().words; }
+
+    void begin_launch() {
+        ops_ = 0;
+        out_.emplace_back();
+        out_.back().lmask = local_;
+        words().reserve(256);
+    }
+
+    // kRunSeg header; its op count is filled in as ops come
+    void begin_segment() {
+        if (words().size() + 2 + run_words(kRunMatAny, R_) > kRunWords - kRunSlack) begin_launch();
+        seg_at_ = (uint32_t)words().size();
+        words().push_back(kRunSeg);
+        words().push_back(compress(rmask_, local_));
+    }
+
+    uint32_t regs(uint32_t mask) const { return compress(mask & rmask_, rmask_); }
+
+    void put_real(double x) {
+        if (R_ == 1) {
+            const float f = (float)x;
+            uint32_t w;
+            std::memcpy(&w, &f, 4);
+            words().push_back(w);
+        } else {
+            uint32_t w[2];
+            std::memcpy(w, &x, 8);
+            words().push_back(w[0]);
+            words().push_back(w[1]);
+        }
+    }
+
+    void put(uint32_t code, uint32_t reg_any_or_all, uint32_t mask, const double* m, int nm, uint32_t all_regs = 0,
+             uint32_t all_mask = 0) {
+        if (words().size() + run_words(code, R_) > kRunWords - kRunSlack) {
+            begin_launch();
+            begin_segment();
+        }
+        words()[seg_at_] += 1u << 8;
+        ++ops_;
+        words().push_back(code | (reg_any_or_all << 8) | (all_regs << 12) | (run_words(code, R_) << 16));
+        words().push_back(mask);
+        if (code >= kRunXAny && code < kRunTerm) words().push_back(all_mask);
+        for (int i = 0; i < nm; ++i) put_real(m[i]);
+    }
+
+    void put_op(const POp& o) {
+        const uint32_t s = compress(o.nd, rmask_);
+        const uint32_t S = (uint32_t)__builtin_ctz(s);
+        const uint32_t ar = regs(o.all), am = o.all & ~rmask_;
+        if (o.any) {
+            const uint32_t yr = regs(o.any), ym = o.any & ~rmask_;
+            if (o.kind == K_X)
+                put(kRunXAny + S, yr, ym, nullptr, 0, ar, am);
+            else
+                put(kRunMatAny + S, yr, ym, o.m, 8, ar, am);
+            return;
+        }
+        switch (o.kind) {
+            case K_MATP: put(kRunMatP + S, 0, 0, o.m, 4); break;
+            case K_REAL: put((o.all ? kRunRealC : kRunReal) + S, ar, am, o.m, 4); break;
+            case K_MAT: put((o.all ? kRunMatC : kRunMat) + S, ar, am, o.m, 8); break;
+            default: put((am ? kRunXC : ar ? kRunXReg : kRunX) + S, ar, am, nullptr, 0); break;
+        }
+    }
+
+    struct Term {
+        uint32_t reg, mask;
+        cd z;
+    };
+    std::vector<Term> terms_;
+
+    // The gathered diagonal ops: terms with equal bits multiplied together,
+    // grouped by register bits.
+    void flush_terms() {
+        if (terms_.empty()) return;
+        std::sort(terms_.begin(), terms_.end(), [](const Term& a, const Term& b) {
+            return a.reg != b.reg ? a.reg < b.reg : a.mask < b.mask;
+        });
+        size_t k = 0;
+        for (size_t i = 0; i < terms_.size();) {
+            Term t = terms_[i++];
+            for (; i < terms_.size() && terms_[i].reg == t.reg && terms_[i].mask == t.mask; ++i) t.z *= terms_[i].z;
+            if (t.z != cd(1)) terms_[k++] = t;
+        }
+        terms_.resize(k);
+        for (size_t i = 0; i < k;) {
+            size_t e = i;
+            bool real = true;
+            for (; e < k && terms_[e].reg == terms_[i].reg; ++e) real = real && terms_[e].z.imag() == 0.0;
+            // a group stays in one launch (its pending factor lives in
+            // registers), or is applied term by term when none holds it
+            const size_t need = (e - i) * run_words(kRunTerm, R_);
+            bool whole = words().size() + need <= kRunWords - kRunSlack;
+            if (!whole && need + 2 <= kRunWords - kRunSlack) {
+                begin_launch();
+                begin_segment();
+                whole = true;
+            }
+            for (; i < e; ++i) {
+                const double z[2] = {terms_[i].z.real(), terms_[i].z.imag()};
+                put(whole && i + 1 < e ? kRunTerm : real ? kRunPhaseReal : kRunPhase, terms_[i].reg, terms_[i].mask, z,
+                    2);
+            }
+        }
+        terms_.clear();
+    }
+
+    void segments(uint32_t local) {
+        local_ = local;
+        begin_launch();
+        while (!members_.empty()) {
+            // slots: the first 4 distinct targets among the ops that are ready
+            uint32_t rm = 0;
+            Passed st;
+            for (uint32_t i : members_) {
+                const POp& o = list_[i];
+                if (st.blocks(o)) {
+                    st.over(o);
+                    continue;
+                }
+                if (__builtin_popcount(rm | o.nd) <= kRunRegBits)
+                    rm |= o.nd;
+                else
+                    st.over(o);
+                if (__builtin_popcount(rm) == kRunRegBits && (st.nd & rm) == rm) break;
+            }
+            // free slots from the top of the tile: neighbouring threads then
+            // hold neighbouring amplitudes
+            for (int b = 31; b >= 0 && __builtin_popcount(rm) < kRunRegBits; --b) rm |= local & (1u << b);
+            rmask_ = rm;
+            begin_segment();
+            st = Passed();
+            left_.clear();
+            uint32_t term_bits = 0;
+            for (uint32_t i : members_) {
+                const POp& o = list_[i];
+                if (st.blocks(o) || (o.nd & ~rm)) {
+                    st.over(o);
+                    left_.push_back(i);
+                    continue;
+                }
+                if (o.kind == K_PHASE) {
+                    terms_.push_back({regs(o.all), o.all & ~rm, cd(o.m[0], o.m[1])});
+                    term_bits |= o.all;
+                } else {
+                    if (o.nd & term_bits) {  // gathered terms that the op does not commute with
+                        flush_terms();
+                        term_bits = 0;
+                    }
+                    put_op(o);
+                }
+            }
+            flush_terms();
+            members_.swap(left_);
+        }
+        if (!ops_) out_.pop_back();  // its gates cancelled exactly
+    }
+};
+
+}  // namespace
+
+namespace aqs_hip {
+
+std::vector<RunLaunch> plan_runs(const aqs_op* ops, size_t count, int n, int m, int precision) {
+    // (a tile smaller than the state holds bits 0..4 and room for a gate's)
+    if (n < 1 || n > kRunMaxQubits || m < 1 || m > n || (m < n && m < 9))
+        fail(AQS_ERR_RUNTIME, "run does not fit the state");
+    // a tile holds at least 16 amplitudes; smaller states are padded with zeros
+    Planner p(std::max(n, kRunRegBits), std::max(m, kRunRegBits), precision);
+    if (n >= kRunRegBits) return p.run(ops, count);
+    std::vector<aqs_op> shifted(ops, ops + count);  // qubits count from the top index bit
+    const int d = kRunRegBits - n;
+    for (aqs_op& o : shifted) {
+        for (int j = 0; j < o.ntargets; ++j) o.targets[j] += d;
+        for (int j = 0; j < o.ncontrols; ++j) o.controls[j] += d;
+        o.more_controls <<= d;
+    }
+    return p.run(shifted.data(), count);
+}
+
+}  // namespace aqs_hip

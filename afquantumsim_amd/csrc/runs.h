@@ -1,0 +1,105 @@
+// Runs of uncompiled ops: what aqs_apply makes of a list of gates on one
+// state.
+//
+// The reference's simulate() (src/quantum.cpp:277-291) applies one operator
+// per gate.  Here a list of ops becomes a few launches, each one sweep of the
+// state in LDS-resident tiles of 2^m amplitudes.  The program of a launch
+// travels in its kernel arguments: nothing is allocated, copied or waited for,
+// and a launch can be captured.  The planner is meant to be cheap (it runs in
+// every call, 0.2-0.4 us per op): bit masks over index bits, no matrices
+// larger than 2 x 2.
+#ifndef AQS_RUNS_H
+#define AQS_RUNS_H
+
+#include <cstddef>
+#include <cstdint>
+#include <vector>
+
+#include "internal.h"
+
+namespace aqs_hip {
+
+constexpr int kRunRegBits = 4;
+constexpr int kRunMaxQubits = 31;      // state indices and masks in 32 bits
+constexpr int kRunMaxTileC64 = 13;     // 67 KiB of LDS: two workgroups per CU
+constexpr int kRunMaxTileC128 = 12;
+
+// A launch's program is a stream of 32-bit words: segments, each a header
+// and its ops.  Word 0 of an op = code | registers << 8 (| registers << 12) |
+// words of the op << 16 (so that the kernel finds the next one at once),
+// word 1 = index-bit mask, then the op's real numbers (one or two words each).
+//   kRunSeg       word 0: code | op count << 8; word 1: the 4 tile-local
+//                 positions that are the threads' register slots (ascending)
+// Ops on the pair of slot S (code + S); controls are slots ("registers") and
+// index bits outside the slots (mask), all of which must be 1:
+//   kRunMatP      the slot's 1-half times (m2, m3), then the rotation by three
+//                 shears (m0 = t, m1 = s); no controls
+//   kRunReal      real 2x2, no controls
+//   kRunRealC     real 2x2 with controls
+//   kRunMat       complex 2x2, no controls
+//   kRunMatC      complex 2x2 with controls
+//   kRunX         exchange; kRunXReg: controls on slots only; kRunXC: any
+//   kRunXAny, kRunMatAny   at least one of (mask, registers) and all of
+//                 (word 2, registers << 12)
+// Diagonal ops: z = m0 + i m1 where all bits of mask and all slots of
+// registers are 1:
+//   kRunTerm      multiplied into the thread's pending factor (mask only)
+//   kRunPhase     the same, then the factor is applied to the amplitudes of
+//                 `registers` and starts again from 1
+//   kRunPhaseReal the same for a group whose factors are all real
+enum : uint32_t {
+    kRunSeg = 0,
+    kRunMatP = 4,
+    kRunReal = 8,
+    kRunRealC = 12,
+    kRunMat = 16,
+    kRunMatC = 20,
+    kRunX = 24,
+    kRunXReg = 28,
+    kRunXC = 32,
+    kRunXAny = 36,
+    kRunMatAny = 40,
+    kRunTerm = 44,
+    kRunPhase = 45,
+    kRunPhaseReal = 46,
+};
+
+// Words of an entry; R words per real number (1 complex64, 2 complex128).
+__host__ __device__ constexpr uint32_t run_words(uint32_t code, uint32_t R) {
+    return code < kRunMatP     ? 2u
+           : code < kRunMat    ? 2u + 4u * R
+           : code < kRunX      ? 2u + 8u * R
+           : code < kRunXAny   ? 2u
+           : code < kRunMatAny ? 3u
+           : code < kRunTerm   ? 3u + 8u * R
+                               : 2u + 2u * R;
+}
+
+// Program words per launch; the kernel reads one entry ahead, so the last
+// kRunSlack words stay unused.  1000 words keep the arguments under 4 KiB.
+constexpr uint32_t kRunWords = 1000;
+constexpr uint32_t kRunSlack = 20;
+
+struct RunLaunch {
+    uint32_t lmask = 0;  // the tile's index bits (m of them, bits 0..min(m, 5)-1 among them)
+    std::vector<uint32_t> words;
+};
+
+// True for ops that runs take (validated; every kind but MATK).
+inline bool run_takes(const aqs_op& op) { return op.kind != AQS_OP_MATK; }
+
+// Plans `count` ops on n qubits (1..kRunMaxQubits) for tiles of 2^m
+// amplitudes (m = n, or 9 <= m < n) as launches, in order.  Runs of one-qubit gates on a
+// qubit are multiplied together (FP64) and split into a rotation and phases
+// that wait for the qubit's next gate; a gate joins a launch, and a segment of
+// it, when the bits it changes are in the tile (the slots) and it commutes
+// with every gate passed over (gates that share only bits both use
+// diagonally commute).
+std::vector<RunLaunch> plan_runs(const aqs_op* ops, size_t count, int n, int m, int precision);
+
+// Applies validated ops that run_takes() through runs (runs.hip).
+void apply_run(aqs_state s, const aqs_op* ops, size_t count);
+
+}  // namespace aqs_hip
+
+#endif

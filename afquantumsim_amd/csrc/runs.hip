@@ -1,0 +1,285 @@
+// Runs of uncompiled ops on one state (runs.h): the kernel and its launches.
+//
+// A workgroup of 2^(m-4) threads (at least one wave) takes a tile of 2^m
+// amplitudes into LDS; per segment every thread holds 16 of them, the
+// combinations of the segment's 4 slot bits, and applies the segment's ops to
+// them in registers, one LDS round trip and one barrier per segment.  A
+// state of at most 2^m amplitudes is one workgroup.
+//
+// What bounds it: on small states the chain of one op after another in each
+// wave (fetch an entry, branch on its code, 40-130 VALU instructions: 0.4 us
+// per op at 12 qubits); entries come through scalar loads from the kernel
+// arguments, and the next entry is loaded while the current one runs.  On
+// large states the VALU, at one sweep of HBM per launch.  Measured against one
+// launch per gate (states of up to 12 qubits: one thread per amplitude pair,
+// a barrier per gate): random layers 12 qubits depth 30 686 -> 266 us, 20 qubits
+// depth 40 6.2 -> 0.84 ms, brickwork 28 qubits depth 4 92.7 -> 9.6 ms, 25 qubits
+// complex128 depth 3 16.6 -> 2.0 ms.
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <cstring>
+
+#include "internal.h"
+#include "regops.h"
+#include "runs.h"
+
+using namespace aqs_hip;
+
+namespace {
+
+struct RunArgs {
+    void* sv;
+    uint32_t n, m;
+    uint32_t lmask;  // index bits of the tile
+    uint32_t words;
+    uint32_t w[kRunWords];
+};
+static_assert(sizeof(RunArgs) <= 4096, "kernel arguments");
+
+// Bits of v (ascending) at the set positions of mask (ascending).
+__device__ __forceinline__ uint32_t deposit(uint32_t v, uint32_t mask) {
+    uint32_t r = 0;
+    for (; mask && v; mask &= mask - 1u, v >>= 1)
+        if (v & 1u) r |= mask & (0u - mask);
+    return r;
+}
+
+// The k-th real number of an entry whose numbers start at word w[0].
+template <typename R>
+__device__ __forceinline__ R real_at(const uint32_t* w, uint32_t k) {
+    if constexpr (sizeof(R) == 4)
+        return __uint_as_float(w[k]);
+    else
+        return __hiloint2double((int)w[2 * k + 1], (int)w[2 * k]);
+}
+
+template <typename T2, typename R, int BS>
+__global__ __launch_bounds__(BS, sizeof(T2) == 8 ? 4 : 2) void k_run(const RunArgs a) {
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+    const uint32_t m = a.m, T = 1u << m, hi_n = m > 5 ? 1u << (m - 5) : 1u;
+    T2* lds = reinterpret_cast<T2*>(smem);
+    uint32_t* hi_tab = reinterpret_cast<uint32_t*>(lds + lds_len(T) + 2);
+    T2* sv = reinterpret_cast<T2*>(a.sv);
+    const uint32_t tid = threadIdx.x, lmask = a.lmask;
+    const uint64_t N = 1ull << a.n;  // below 16 amplitudes the tile is padded with zeros
+    // index bits of the tile's positions 5.. and of the tile itself
+    for (uint32_t v = tid; v < hi_n; v += BS) hi_tab[v] = deposit(v, lmask & ~31u);
+    const uint32_t base = deposit(blockIdx.x, (uint32_t)(N - 1u) & ~lmask);
+    __syncthreads();
+    constexpr uint32_t A = sizeof(T2) == 8 ? 2 : 1;  // amplitudes per 16-byte unit
+    for (uint32_t l = A * tid; l < T; l += A * BS) {
+        const uint32_t g = base | (l & 31u) | hi_tab[l >> 5];
+        float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (g < N) v = reinterpret_cast<const float4*>(sv)[g / A];
+        *reinterpret_cast<float4*>(&lds[lds_pad(l)]) = v;
+    }
+    __syncthreads();
+    const uint32_t groups = T >> kRunRegBits;
+    // the entry that comes next: its two words and numbers, loaded while the
+    // current one runs
+    uint32_t at = 0, n0 = a.w[0], n1 = a.w[1];
+    R nc[8];
+    R fr = R(1), fi = R(0);  // the thread's pending factor
+    while (at < a.words) {
+        // segment header
+        const uint32_t nops = n0 >> 8, rmask = n1;
+        at += 2;
+        n0 = a.w[at];
+        n1 = a.w[at + 1];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) nc[k] = real_at<R>(a.w + at + 2, k);
+        const uint32_t r0 = rmask & (0u - rmask), rm1 = rmask & (rmask - 1u), r1 = rm1 & (0u - rm1),
+                       rm2 = rm1 & (rm1 - 1u), r2 = rm2 & (0u - rm2), r3 = rm2 & (rm2 - 1u);
+        // thread -> tile position with zeros at the slots (ascending), and
+        // that position's state index
+        uint32_t lt = tid;
+        lt = ((lt & ~(r0 - 1u)) << 1) | (lt & (r0 - 1u));
+        lt = ((lt & ~(r1 - 1u)) << 1) | (lt & (r1 - 1u));
+        lt = ((lt & ~(r2 - 1u)) << 1) | (lt & (r2 - 1u));
+        lt = ((lt & ~(r3 - 1u)) << 1) | (lt & (r3 - 1u));
+        const bool live = tid < groups;
+        if (!live) lt = 0;
+        const uint32_t idx = base | (lt & 31u) | hi_tab[lt >> 5];
+        const uint32_t p0 = lds_pad(lt);
+        auto slot = [&](int j) {
+            return p0 + lds_pad(((j & 1) ? r0 : 0u) | ((j & 2) ? r1 : 0u) | ((j & 4) ? r2 : 0u) | ((j & 8) ? r3 : 0u));
+        };
+        T2 x[16];
+#pragma unroll
+        for (int j = 0; j < 16; ++j) x[j] = lds[slot(j)];
+        for (uint32_t o = 0; o < nops; ++o) {
+            const uint32_t c0 = n0, mask = n1, here = at;
+            const uint32_t code = c0 & 255u, creg = (c0 >> 8) & 15u;
+            R c[8];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) c[k] = nc[k];
+            at += c0 >> 16;
+            n0 = a.w[at];
+            n1 = a.w[at + 1];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) nc[k] = real_at<R>(a.w + at + 2, k);
+            const bool thr = (idx & mask) == mask;
+            auto all_ok = [&](int j) { return thr && ((uint32_t)j & creg) == creg; };
+            if (code >= kRunTerm) {
+                const R zr = thr ? c[0] : R(1), zi = thr ? c[1] : R(0);
+                cmul_acc(fr, fi, zr, zi);
+                if (code == kRunTerm) continue;
+                if (code == kRunPhaseReal) {
+                    switch (creg) {
+#define AQS_REAL_CASE(M)                                                       \
+    case M:                                                                    \
+        _Pragma("unroll") for (int j = 0; j < 16; ++j) if ((j & (M)) == (M)) { \
+            x[j].x *= fr;                                                      \
+            x[j].y *= fr;                                                      \
+        }                                                                      \
+        break;
+                        AQS_REAL_CASE(0) AQS_REAL_CASE(1) AQS_REAL_CASE(2) AQS_REAL_CASE(3)
+                        AQS_REAL_CASE(4) AQS_REAL_CASE(5) AQS_REAL_CASE(6) AQS_REAL_CASE(7)
+                        AQS_REAL_CASE(8) AQS_REAL_CASE(9) AQS_REAL_CASE(10) AQS_REAL_CASE(11)
+                        AQS_REAL_CASE(12) AQS_REAL_CASE(13) AQS_REAL_CASE(14)
+#undef AQS_REAL_CASE
+                        default:  // mask 15
+                            x[15].x *= fr;
+                            x[15].y *= fr;
+                            break;
+                    }
+                } else {
+                    switch (creg) {
+#define AQS_MASK_CASE(M)                                                       \
+    case M:                                                                    \
+        _Pragma("unroll") for (int j = 0; j < 16; ++j) if ((j & (M)) == (M))   \
+            x[j] = cmul<T2, R>(fr, fi, x[j]);                                  \
+        break;
+                        AQS_MASK_CASE(0) AQS_MASK_CASE(1) AQS_MASK_CASE(2) AQS_MASK_CASE(3)
+                        AQS_MASK_CASE(4) AQS_MASK_CASE(5) AQS_MASK_CASE(6) AQS_MASK_CASE(7)
+                        AQS_MASK_CASE(8) AQS_MASK_CASE(9) AQS_MASK_CASE(10) AQS_MASK_CASE(11)
+                        AQS_MASK_CASE(12) AQS_MASK_CASE(13) AQS_MASK_CASE(14)
+#undef AQS_MASK_CASE
+                        default:  // mask 15
+                            x[15] = cmul<T2, R>(fr, fi, x[15]);
+                            break;
+                    }
+                }
+                fr = R(1);
+                fi = R(0);
+                continue;
+            }
+            const R mp[8] = {c[0], c[1], R(0), R(0), c[2], c[3], R(0), R(0)};
+            switch (code) {
+#define AQS_RUN(C, SL, OP, FORM, MAT, OK) \
+    case C + SL: pairs<SL, OP, FORM>(x, MAT, creg, OK); break;
+#define AQS_RUN4(C, OP, FORM, MAT, OK)                                        \
+    AQS_RUN(C, 0, OP, FORM, MAT, OK) AQS_RUN(C, 1, OP, FORM, MAT, OK)         \
+    AQS_RUN(C, 2, OP, FORM, MAT, OK) AQS_RUN(C, 3, OP, FORM, MAT, OK)
+                AQS_RUN4(kRunMatP, 3, 0, mp, all_ok)
+                AQS_RUN4(kRunReal, 2, 0, c, all_ok)
+                AQS_RUN4(kRunRealC, 2, 2, c, all_ok)
+                AQS_RUN4(kRunMat, 0, 0, c, all_ok)
+                AQS_RUN4(kRunMatC, 0, 2, c, all_ok)
+                AQS_RUN4(kRunX, 1, 0, c, all_ok)
+                AQS_RUN4(kRunXReg, 1, 1, c, all_ok)
+                AQS_RUN4(kRunXC, 1, 2, c, all_ok)
+#undef AQS_RUN4
+#undef AQS_RUN
+                default: {  // any-of forms: a third word, then the numbers
+                    const uint32_t areg = (c0 >> 12) & 15u, amask = a.w[here + 2];
+                    const bool athr = (idx & amask) == amask, some = (idx & mask) != 0u;
+                    auto any_ok = [&](int j) {
+                        return (some || ((uint32_t)j & creg) != 0u) && athr && ((uint32_t)j & areg) == areg;
+                    };
+                    R d[8];
+#pragma unroll
+                    for (int k = 0; k < 8; ++k) d[k] = real_at<R>(a.w + here + 3, k);
+                    switch (code) {
+                        case kRunXAny: pairs<0, 1, 2>(x, d, creg, any_ok); break;
+                        case kRunXAny + 1: pairs<1, 1, 2>(x, d, creg, any_ok); break;
+                        case kRunXAny + 2: pairs<2, 1, 2>(x, d, creg, any_ok); break;
+                        case kRunXAny + 3: pairs<3, 1, 2>(x, d, creg, any_ok); break;
+                        case kRunMatAny: pairs<0, 0, 2>(x, d, creg, any_ok); break;
+                        case kRunMatAny + 1: pairs<1, 0, 2>(x, d, creg, any_ok); break;
+                        case kRunMatAny + 2: pairs<2, 0, 2>(x, d, creg, any_ok); break;
+                        default: pairs<3, 0, 2>(x, d, creg, any_ok); break;
+                    }
+                    break;
+                }
+            }
+        }
+        if (live) {
+#pragma unroll
+            for (int j = 0; j < 16; ++j) lds[slot(j)] = x[j];
+        }
+        __syncthreads();
+    }
+    for (uint32_t l = A * tid; l < T; l += A * BS) {
+        const uint32_t g = base | (l & 31u) | hi_tab[l >> 5];
+        if (g < N) reinterpret_cast<float4*>(sv)[g / A] = *reinterpret_cast<const float4*>(&lds[lds_pad(l)]);
+    }
+}
+
+template <typename T2, typename R, int BS>
+void launch_bs(aqs_state s, const RunArgs& a) {
+    const size_t tile = (size_t)1 << a.m;
+    const size_t lds = (lds_len(tile) + 2) * sizeof(T2) + (std::max<size_t>(tile >> 5, 1)) * sizeof(uint32_t);
+    if (lds > 65536) {
+        static std::once_flag once;
+        static hipError_t rc = hipSuccess;
+        std::call_once(once, [] {
+            rc = hipFuncSetAttribute((const void*)k_run<T2, R, BS>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                     80 * 1024);
+        });
+        AQS_HIP(rc);
+    }
+    const uint64_t tiles = s->n > (int)a.m ? s->N >> a.m : 1;
+    ProfScope ps(s, kSlotRuns);
+    hipLaunchKernelGGL((k_run<T2, R, BS>), dim3((unsigned)tiles), dim3(BS), lds, s->stream, a);
+    AQS_HIP(hipGetLastError());
+}
+
+template <typename T2, typename R>
+void launch_run(aqs_state s, const RunArgs& a) {
+    switch (a.m) {
+        case 13: launch_bs<T2, R, 512>(s, a); break;
+        case 12: launch_bs<T2, R, 256>(s, a); break;
+        case 11: launch_bs<T2, R, 128>(s, a); break;
+        default: launch_bs<T2, R, 64>(s, a); break;
+    }
+}
+
+}  // namespace
+
+namespace aqs_hip {
+
+// Tile of a run.  A state of up to 12 (complex64) or 11 (complex128) qubits is
+// one tile.  Above, smaller tiles spread a medium state over more CUs and
+// leave each wave alone on its SIMD, larger ones take more gates per launch;
+// measured (random layers, depth 40, us by tile of 10 / 11 / 12 / 13 qubits):
+// 13 qubits 378 / 336 / 338 / 405, 17 qubits 566 / 541 / 578 / 670, 19 qubits
+// 713 / 648 / 662 / 800, 20 qubits 956 / 965 / 833 / 944; brickwork depth 10:
+// 22 qubits 418 / 364 / 350 / 328.  complex128, depth 20, 10 / 11 / 12: 16
+// qubits 336 / 333 / 377, 20 qubits 726 / 718 / 616.
+static int run_tile_qubits(int n, int precision) {
+    if (precision == AQS_C64) return n <= 12 ? n : n <= 16 ? 12 : n <= 19 ? 11 : n == 20 ? 12 : kRunMaxTileC64;
+    return n <= 11 ? n : n <= 18 ? 11 : kRunMaxTileC128;
+}
+
+void apply_run(aqs_state s, const aqs_op* ops, size_t count) {
+    const int m = run_tile_qubits(s->n, s->precision);
+    for (const RunLaunch& l : plan_runs(ops, count, s->n, m, s->precision)) {
+        RunArgs a;
+        a.sv = s->amps;
+        a.n = (uint32_t)s->n;
+        a.m = (uint32_t)std::max(m, kRunRegBits);
+        a.lmask = l.lmask;
+        a.words = (uint32_t)l.words.size();
+        if (a.words > kRunWords - kRunSlack) fail(AQS_ERR_RUNTIME, "run program too long");
+        std::memcpy(a.w, l.words.data(), l.words.size() * sizeof(uint32_t));
+        std::memset(a.w + a.words, 0, (kRunWords - a.words) * sizeof(uint32_t));
+        if (s->precision == AQS_C64)
+            launch_run<float2, float>(s, a);
+        else
+            launch_run<double2, double>(s, a);
+    }
+}
+
+}  // namespace aqs_hip

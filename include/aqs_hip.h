@@ -145,9 +145,12 @@ aqs_status aqs_state_download(aqs_state s, void* host);
 
 /* ---- gate application (QSimulator::simulate, src/quantum.cpp:277-291) --- */
 
-/* Apply ops in order, one HIP kernel pass each; on a state of at most 12
- * qubits (complex64) or 11 (complex128), runs of two or more non-MATK ops
- * are applied by one LDS-resident workgroup, up to 64 (40) ops per launch. */
+/* Apply ops in order.  A call's runs of two or more non-MATK ops (states of
+ * at most 31 qubits) go through LDS-resident tiles, many ops per sweep of the
+ * state; on a state of at most 12 qubits (complex64) or 11 (complex128) up to
+ * 64 (40) ops per launch of one workgroup.  A single op, MATK ops and, from 20
+ * qubits up, lists that touch less than 1.5 times the state in all (a few
+ * phases or controlled flips) are one HIP kernel pass per op. */
 aqs_status aqs_apply(aqs_state s, const aqs_op* ops, size_t count);
 
 /* Launch-shape autotuner for the one-qubit pass at this state's size: times
@@ -341,7 +344,7 @@ aqs_status aqs_profile_enable(aqs_state s, int enable);
 /* Slots (arrays of AQS_PROFILE_SLOTS): 0 state preparation and measurement,
  * 1..6 the AQS_OP_* kind of a plain pass (MATK on the scalar kernel), 7 MATK
  * on MFMA, 8 diagonal table passes, 9 bit-permutation passes, 10 tile
- * passes, 11 runs of ops on a small state held in LDS (aqs_apply).  Total ms
+ * passes, 11 runs of ops in LDS tiles (aqs_apply).  Total ms
  * and launch count since enable. */
 #define AQS_PROFILE_SLOTS 12
 aqs_status aqs_profile_read(aqs_state s, double* ms_by_kind, uint64_t* launches_by_kind);

@@ -7,7 +7,8 @@
 // segment, per thread the 16 register amplitudes, with the op encodings
 // (register slots, thread-fixed positions, global bits) interpreted as the
 // kernel interprets them.  Plain passes and bit permutations are applied
-// directly.  batch_emulate() runs the program of one batched state
+// directly.  run_emulate() runs the launches of aqs_apply's runs
+// (afquantumsim_amd/csrc/runs.hip) word by word.  batch_emulate() runs the program of one batched state
 // (afquantumsim_amd/csrc/batch.hip) phase by phase and tile by tile.
 // block_emulate() does the same for the dense-block schedule of
 // aqs_fuse, diagonal tables included (afquantumsim_amd/csrc/diag.hip:
@@ -19,6 +20,7 @@
 #include <vector>
 
 #include "batch.h"
+#include "runs.h"
 #include "schedule.h"
 
 using namespace aqs_hip;
@@ -506,6 +508,137 @@ int batch_emulate(const aqs_op* ops, size_t count, int n, int m, double* state, 
     counts[1] = phases.size();
     counts[2] = loads;
     counts[3] = reg_segs;
+    return AQS_OK;
+}
+
+// Plans the ops as runs for tiles of 2^m amplitudes (m >= 4, n >= m) and
+// applies the launches to `state` (2^n complex FP64) on the host: per tile, per
+// segment, per thread the 16 amplitudes of its slots, entry by entry as
+// k_run reads them.  Negative on a program that the kernel could not run
+// (entries past the end, slots or masks out of range, a pending factor left
+// over).  counts[0..2] = launches, segments, entries.
+int run_emulate(const aqs_op* ops, size_t count, int n, int m, int precision, double* state, size_t* counts) {
+    std::vector<RunLaunch> launches;
+    try {
+        launches = plan_runs(ops, count, n, m, precision);
+    } catch (...) {
+        return -1;
+    }
+    n = n < kRunRegBits ? kRunRegBits : n;  // the kernel pads smaller states with zeros
+    m = m < kRunRegBits ? kRunRegBits : m;
+    const size_t N = (size_t)1 << n, N_state = counts[3];
+    std::vector<cplx> v(N);
+    std::memcpy(v.data(), state, N_state * sizeof(cplx));
+    const uint32_t RW = precision == AQS_C64 ? 1 : 2;
+    counts[0] = launches.size();
+    counts[1] = counts[2] = 0;
+    auto real = [&](const uint32_t* w, int k) {
+        if (RW == 1) {
+            float f;
+            std::memcpy(&f, w + k, 4);
+            return (double)f;
+        }
+        double d;
+        std::memcpy(&d, w + 2 * k, 8);
+        return d;
+    };
+    for (const RunLaunch& l : launches) {
+        if (l.words.size() > kRunWords - kRunSlack || __builtin_popcount(l.lmask) != m || (n < 32 && (l.lmask >> n)))
+            return -2;
+        if ((l.lmask & ((1u << (m < 5 ? m : 5)) - 1u)) != (1u << (m < 5 ? m : 5)) - 1u) return -3;
+        std::vector<int> loc, out;
+        for (int b = 0; b < n; ++b) ((l.lmask >> b) & 1u ? loc : out).push_back(b);
+        for (size_t at = 0; at < l.words.size();) {
+            if ((l.words[at] & 255u) != kRunSeg || at + 2 > l.words.size()) return -4;
+            const uint32_t nops = l.words[at] >> 8, rmask = l.words[at + 1];
+            at += 2;
+            ++counts[1];
+            if (__builtin_popcount(rmask) != 4 || (rmask >> m)) return -5;
+            uint32_t rbits = 0;
+            std::vector<int> slot;
+            for (int p = 0; p < m; ++p)
+                if ((rmask >> p) & 1u) {
+                    slot.push_back(loc[p]);
+                    rbits |= 1u << loc[p];
+                }
+            size_t end = at;
+            for (size_t g = 0; g < (N >> 4); ++g) {  // every thread of every tile
+                uint32_t idx = 0;
+                size_t bits = g;
+                for (int b = 0; b < n; ++b)
+                    if (!((rbits >> b) & 1u)) {
+                        idx |= (uint32_t)(bits & 1u) << b;
+                        bits >>= 1;
+                    }
+                auto amp = [&](int j) -> cplx& {
+                    uint32_t i = idx;
+                    for (int q = 0; q < 4; ++q)
+                        if ((j >> q) & 1) i |= 1u << slot[q];
+                    return v[i];
+                };
+                cplx f(1);
+                end = at;
+                for (uint32_t o = 0; o < nops; ++o) {
+                    if (end >= l.words.size()) return -6;
+                    const uint32_t* w = l.words.data() + end;
+                    const uint32_t code = w[0] & 255u, creg = (w[0] >> 8) & 15u, mask = w[1];
+                    if (code < kRunMatP || code > kRunPhaseReal || (n < 32 && (mask >> n)) || (mask & rbits)) return -7;
+                    if ((w[0] >> 16) != run_words(code, RW)) return -12;
+                    end += w[0] >> 16;
+                    if (end > l.words.size()) return -8;
+                    const bool thr = (idx & mask) == mask;
+                    if (code >= kRunTerm) {
+                        if (thr) f *= cplx(real(w + 2, 0), real(w + 2, 1));
+                        if (code == kRunTerm) continue;
+                        if (code == kRunPhaseReal && f.imag() != 0.0) return -9;
+                        for (int j = 0; j < 16; ++j)
+                            if (((uint32_t)j & creg) == creg) amp(j) *= f;
+                        f = cplx(1);
+                        continue;
+                    }
+                    const bool any = code >= kRunXAny;
+                    const uint32_t areg = (w[0] >> 12) & 15u, amask = any ? w[2] : 0u;
+                    const uint32_t family = code & ~3u;
+                    const int S = 1 << (code & 3u);
+                    if ((creg | areg) & (uint32_t)S) return -10;
+                    for (int j = 0; j < 16; ++j) {
+                        if (j & S) continue;
+                        bool ok = true;
+                        if (any)
+                            ok = ((idx & mask) || ((uint32_t)j & creg)) && (idx & amask) == amask &&
+                                 ((uint32_t)j & areg) == areg;
+                        else if (family == kRunRealC || family == kRunMatC || family == kRunXC)
+                            ok = thr && ((uint32_t)j & creg) == creg;
+                        else if (family == kRunXReg)
+                            ok = ((uint32_t)j & creg) == creg;
+                        if (!ok) continue;
+                        cplx &x = amp(j), &y = amp(j | S);
+                        const cplx p = x, q = y;
+                        const uint32_t* r = w + (any ? 3 : 2);
+                        if (family == kRunMatP) {
+                            const cplx z = q * cplx(real(r, 2), real(r, 3));
+                            const cplx p1 = p - real(r, 0) * z, q1 = z + real(r, 1) * p1;
+                            x = p1 - real(r, 0) * q1;
+                            y = q1;
+                        } else if (family == kRunReal || family == kRunRealC) {
+                            x = real(r, 0) * p + real(r, 1) * q;
+                            y = real(r, 2) * p + real(r, 3) * q;
+                        } else if (family == kRunMat || family == kRunMatC || family == kRunMatAny) {
+                            x = cplx(real(r, 0), real(r, 1)) * p + cplx(real(r, 2), real(r, 3)) * q;
+                            y = cplx(real(r, 4), real(r, 5)) * p + cplx(real(r, 6), real(r, 7)) * q;
+                        } else {
+                            x = q;
+                            y = p;
+                        }
+                    }
+                }
+                if (f != cplx(1)) return -11;
+            }
+            counts[2] += nops;
+            at = end;
+        }
+    }
+    std::memcpy(state, v.data(), N_state * sizeof(cplx));
     return AQS_OK;
 }
 

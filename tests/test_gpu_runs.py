@@ -1,0 +1,78 @@
+"""Runs of uncompiled ops on the GPU (aqs_apply on a list of ops) at the sizes
+where the tile changes, against the per-op kernels (one aqs_apply per op) and
+the numpy restatement."""
+import numpy as np
+import pytest
+
+from afquantumsim_amd import hip
+from tests.helpers import random_state
+from tests.test_batch_cpu import batch_ops
+from tests.test_gpu_small import mixed_ops, np_run_any
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module", autouse=True)
+def _device():
+    hip.init(0)
+    yield
+
+
+def apply(n, precision, sv, op_list):
+    st = hip.State(n, precision)
+    st.upload(sv.astype(st.dtype))
+    st.profile(True)
+    st.apply(op_list)
+    prof = st.profile_read()
+    got = st.download()
+    st.close()
+    return got, prof
+
+
+CASES = [(hip.C64, n) for n in (4, 6, 11, 12, 13, 16, 17, 19, 20, 21)] + [(hip.C128, n) for n in (5, 11, 12, 18, 19)]
+
+
+@pytest.mark.parametrize("precision,n", CASES, ids=[f"{'c64' if p == hip.C64 else 'c128'}-{n}q" for p, n in CASES])
+def test_runs_match_restatement(precision, n):
+    """Every op kind, one-qubit runs that merge, many controls.  At most 160
+    gates: FP32 rounding of 160 sequential products stays below 160 x 2^-24 =
+    1e-5 of the norm, an amplitude far below; FP64 likewise 2e-14."""
+    op_list = mixed_ops(n, 90, 3 * n) + batch_ops(n, 40, n)[n:]
+    sv = random_state(n, n)
+    got, prof = apply(n, precision, sv, op_list)
+    assert set(prof) == {"SMALL"}, prof
+    np.testing.assert_allclose(got, np_run_any(sv.astype(np.complex64 if precision == hip.C64 else complex).astype(complex),
+                                               n, op_list), atol=5e-6 if precision == hip.C64 else 1e-12, rtol=0)
+
+
+@pytest.mark.parametrize("precision,n", [(hip.C64, 13), (hip.C64, 18), (hip.C128, 14)])
+def test_permutation_runs_bit_exact(precision, n):
+    op_list = mixed_ops(n, 120, n, perm_only=True)
+    sv = random_state(n, 1)
+    st = hip.State(n, precision)
+    sv = sv.astype(st.dtype)
+    st.close()
+    got, _ = apply(n, precision, sv, op_list)
+    want = np_run_any(sv.astype(complex), n, op_list).astype(sv.dtype)
+    assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+
+
+def test_few_sparse_ops_keep_their_kernels():
+    """From 20 qubits up a list that touches little of the state runs op by op."""
+    n = 20
+    op_list = [{"kind": hip.OP_PHASE, "targets": (a,), "controls": (a + 1,), "m": np.array([-1, 0, 0, 0])} for a in (0, 2, 4)]
+    sv = random_state(n, 2)
+    got, prof = apply(n, hip.C64, sv, op_list)
+    assert set(prof) == {"PHASE"} and prof["PHASE"][1] == 3, prof
+    np.testing.assert_allclose(got, np_run_any(sv, n, op_list), atol=1e-6, rtol=0)
+
+
+def test_error_applies_the_prefix_on_a_tiled_state():
+    n = 14
+    op_list = [{"kind": hip.OP_X, "targets": (0,)}, {"kind": hip.OP_X, "targets": (3,)},
+               {"kind": hip.OP_X, "targets": (n,)}, {"kind": hip.OP_X, "targets": (1,)}]
+    st = hip.State(n, hip.C64)
+    with pytest.raises(hip.OutOfRange):
+        st.apply(op_list)
+    assert abs(st.amplitude((1 << (n - 1)) | (1 << (n - 4))) - 1) == 0
+    st.close()

@@ -1,0 +1,107 @@
+"""Runs of uncompiled ops on the CPU (no GPU): the launches that aqs_apply
+plans (afquantumsim_amd/csrc/runs.cpp), read word by word the way the kernel
+reads them (tests/cpp/tile_emu.cpp, run_emulate), against the numpy
+restatement of every op kind.  complex128 programs agree to 1e-12; complex64
+programs hold matrices rounded to FP32 and agree to 1e-5; permutations bit
+for bit."""
+import ctypes
+import os
+
+import numpy as np
+import pytest
+
+from afquantumsim_amd import circuits, hip, ops
+from tests.helpers import random_state
+from tests.test_batch_cpu import batch_ops
+from tests.test_gpu_small import mixed_ops, np_run_any
+from tests.test_tiling import EMU
+
+
+@pytest.fixture(scope="module")
+def emu():
+    if not os.path.exists(EMU):
+        pytest.fail("tests/cpp/libtile_emu.so is not built (run __graft_entry__.build())")
+    hip.load()
+    lib = ctypes.CDLL(EMU)
+    lib.run_emulate.restype = ctypes.c_int
+    lib.run_emulate.argtypes = [ctypes.POINTER(hip.Op), ctypes.c_size_t, ctypes.c_int, ctypes.c_int, ctypes.c_int,
+                                ctypes.c_void_p, ctypes.POINTER(ctypes.c_size_t)]
+    return lib
+
+
+def emulate(emu, op_list, n, m, precision, sv):
+    p = hip.PackedOps(op_list)
+    v = np.ascontiguousarray(sv, dtype=np.complex128).copy()
+    counts = (ctypes.c_size_t * 4)(0, 0, 0, 1 << n)
+    rc = emu.run_emulate(p.arr, p.count, n, m, precision, v.ctypes.data, counts)
+    assert rc == 0, rc
+    return v, list(counts)[:3]
+
+
+SHAPES = [(1, 1), (2, 2), (3, 3), (4, 4), (5, 5), (6, 6), (9, 9), (12, 12), (10, 9), (12, 10), (14, 11)]
+
+
+@pytest.mark.parametrize("precision,tol", [(hip.C64, 1e-5), (hip.C128, 1e-12)], ids=["c64", "c128"])
+@pytest.mark.parametrize("n,m", SHAPES, ids=[f"{n}q-tile{m}" for n, m in SHAPES])
+def test_every_op_kind(emu, n, m, precision, tol):
+    for seed in (1, 2):
+        op_list = mixed_ops(n, 120, seed + 10 * n)
+        sv = random_state(n, seed)
+        got, _ = emulate(emu, op_list, n, m, precision, sv)
+        np.testing.assert_allclose(got, np_run_any(sv, n, op_list), atol=tol, rtol=0)
+
+
+@pytest.mark.parametrize("n,m", [(6, 6), (11, 9), (13, 10)])
+def test_absorbed_and_many_controlled_ops(emu, n, m):
+    """One-qubit runs that merge, gates with up to six controls, swaps under
+    all-of and any-of controls."""
+    op_list = batch_ops(n, 200, 7 + n)
+    sv = random_state(n, n)
+    got, _ = emulate(emu, op_list, n, m, hip.C128, sv)
+    np.testing.assert_allclose(got, np_run_any(sv, n, op_list), atol=1e-12, rtol=0)
+
+
+@pytest.mark.parametrize("n,m", [(3, 3), (8, 8), (12, 9)])
+def test_permutations_bit_exact(emu, n, m):
+    op_list = mixed_ops(n, 150, 60 + n, perm_only=True)
+    sv = random_state(n, 5)
+    got, _ = emulate(emu, op_list, n, m, hip.C64, sv)
+    assert np.array_equal(got, np_run_any(sv, n, op_list))
+
+
+@pytest.mark.parametrize("name", ["brickwork", "layers", "qft", "iqft"])
+@pytest.mark.parametrize("n,m", [(10, 10), (14, 12)])
+def test_circuits(emu, name, n, m):
+    gates = {"brickwork": lambda: circuits.brickwork(n, 6), "layers": lambda: circuits.random_layered(n, 8),
+             "qft": lambda: circuits.fourier_transform(n), "iqft": lambda: circuits.inverse_fourier_transform(n)}[name]()
+    op_list = ops.lower_all(gates)
+    sv = random_state(n, 3)
+    got, (launches, _, _) = emulate(emu, op_list, n, m, hip.C64, sv)
+    np.testing.assert_allclose(got, np_run_any(sv, n, op_list), atol=1e-5, rtol=0)
+    assert launches < len(op_list) / 8
+
+
+@pytest.mark.parametrize("precision,chunk", [(hip.C64, 64), (hip.C128, 40)], ids=["c64", "c128"])
+def test_one_launch_per_chunk(emu, precision, chunk):
+    """A chunk of ops on a one-tile state fits one launch, whatever its ops."""
+    n = 11
+    rng = np.random.default_rng(0)
+    for seed in range(40):
+        op_list = mixed_ops(n, chunk, seed)
+        if seed % 4 == 0:  # any-of controlled 2x2 gates: the longest entries
+            q = [rng.permutation(n)[:3] for _ in range(chunk)]
+            op_list = [{"kind": hip.OP_MAT1, "targets": (int(a[0]),), "controls": (int(a[1]), int(a[2])),
+                        "flags": hip.CTRL_ANY, "m": rng.normal(size=4) + 1j * rng.normal(size=4)} for a in q]
+        _, (launches, _, _) = emulate(emu, op_list, n, n, precision, np.zeros(1 << n))
+        assert launches <= 1
+
+
+def test_long_phase_groups_split(emu):
+    """More diagonal terms than one launch holds."""
+    n = 13
+    rng = np.random.default_rng(4)
+    op_list = [{"kind": hip.OP_PHASE, "targets": tuple(int(x) for x in rng.permutation(n)[:int(rng.integers(1, 6))]),
+                "m": np.array([np.exp(1j * rng.uniform(-3, 3)), 0, 0, 0])} for _ in range(900)]
+    sv = random_state(n, 8)
+    got, _ = emulate(emu, op_list, n, 12, hip.C128, sv)
+    np.testing.assert_allclose(got, np_run_any(sv, n, op_list), atol=1e-12, rtol=0)

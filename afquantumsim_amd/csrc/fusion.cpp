@@ -940,6 +940,7 @@ aqs_status aqs_fuse(const aqs_op* ops, size_t count, int nqubits, int max_qubits
 aqs_status aqs_schedule_destroy(aqs_schedule sch) {
     return guard([&] {
         if (!sch) return;
+        if (sch->tile_form) aqs_schedule_destroy(sch->tile_form);
         if (sch->dev) (void)hipFree(sch->dev);
         delete sch;
     });
@@ -966,6 +967,7 @@ aqs_status aqs_apply_schedule(aqs_state s, aqs_schedule sch) {
         if (!s || !s->amps) fail(AQS_ERR_INVALID_ARGUMENT, "null state handle");
         if (!sch) fail(AQS_ERR_INVALID_ARGUMENT, "null schedule");
         if (sch->n != s->n) fail(AQS_ERR_INVALID_ARGUMENT, "schedule and state qubit counts differ");
+        if (sch->tile_form) sch = sch->tile_form;
         if (sch->dev_precision != s->precision) {
             // Device copies of the pass data, in the layout each kernel reads:
             // MFMA-packed FP32 (complex64, k = 4, 5), plain FP32 / FP64
@@ -988,7 +990,7 @@ aqs_status aqs_apply_schedule(aqs_state s, aqs_schedule sch) {
             for (size_t p = 0; p < sch->passes.size(); ++p) {
                 const aqs_op& op = sch->passes[p];
                 if (sch->tile_index[p] >= 0) {
-                    const auto& t = sch->tiles[sch->tile_index[p]];
+                    const auto& t = sch->tile(sch->tile_index[p], s->precision);
                     auto& o = sch->dev_tile[p];
                     o[0] = append(t.segs.data(), t.segs.size() * sizeof(TileSegDev));
                     o[1] = append(t.ops.data(), t.ops.size() * sizeof(TileOpDev));
@@ -999,6 +1001,9 @@ aqs_status aqs_apply_schedule(aqs_state s, aqs_schedule sch) {
                         o[3] = append(t.m128.data(), t.m128.size() * sizeof(double));
                         o[4] = append(t.z128.data(), t.z128.size() * sizeof(double));
                         o[7] = append(t.fold_z128.data(), t.fold_z128.size() * sizeof(double));
+                    } else if (!t.dense.empty()) {
+                        const std::vector<uint16_t> d = pack_dense(t.dense);
+                        o[8] = append(d.data(), d.size() * sizeof(uint16_t));
                     }
                     continue;
                 }
@@ -1044,9 +1049,9 @@ aqs_status aqs_apply_schedule(aqs_state s, aqs_schedule sch) {
             if (sch->tile_index[p] >= 0) {
                 const auto& o = sch->dev_tile[p];
                 const char* base = (const char*)sch->dev;
-                apply_tile_pass(s, sch->tiles[sch->tile_index[p]],
+                apply_tile_pass(s, sch->tile(sch->tile_index[p], s->precision),
                                 TileDevProgram{base + o[0], base + o[1], base + o[2], base + o[3], base + o[4],
-                                               base + o[5], base + o[6], base + o[7]});
+                                               base + o[5], base + o[6], base + o[7], base + o[8]});
                 continue;
             }
             if (sch->diag_index[p] >= 0) {

@@ -55,7 +55,8 @@ constexpr int kTileCodePhases = 24;
 constexpr int kTileCodeMatR = 26;
 constexpr int kTileCodeMatP = 38;
 constexpr int kTileCodeMatPSet = 42;
-constexpr int kTileCodeCount = 58;
+constexpr int kTileCodeDense = 58;  // complex64 programs only: see TilePass::dense
+constexpr int kTileCodeCount = 59;
 inline int tile_code(int kind, int form, int slot, bool zeta) {
     if (kind == TILE_PHASES) return kTileCodePhases + (zeta ? 1 : 0);
     if (kind == TILE_MATP) return form == 0 ? kTileCodeMatP + slot : -1;
@@ -145,7 +146,18 @@ struct TilePass {
     std::vector<TileFoldDev> folds;
     std::vector<TileFoldTermDev> fold_terms;
     std::vector<double> fold_z128;  // [fold_terms][2]
+    // Dense ops (kTileCodeDense, term_begin = number): a run of the pass's
+    // gates on 4 local positions multiplied into one 16 x 16 unitary
+    // (row-major, interleaved, FP64).  Bits 0..2 of its index are the
+    // segment's slots 0..2, bit 3 is thread bit 5 (local position thr[5]).
+    std::vector<double> dense;  // [dense][16][16][2]
 };
+constexpr size_t kDenseDoubles = 512;
+
+// The matrix-core operand of dense ops: each unitary as a real 32 x 32
+// matrix, split exactly into three bf16 planes.
+std::vector<uint16_t> pack_dense(const std::vector<double>& dense);
+constexpr size_t kDenseOperand = 3 * 2 * 64 * 8;  // bf16 words of one op
 
 // Device copies of one tile pass's program.
 struct TileDevProgram {
@@ -157,6 +169,7 @@ struct TileDevProgram {
     const void* folds;
     const void* fold_terms;
     const void* fold_z128;
+    const void* dense;
 };
 
 // Runs one tile pass.
@@ -175,11 +188,20 @@ struct aqs_schedule_s {
     std::vector<std::vector<int>> perms;          // bit involutions (AQS_OP_PERMB passes)
     std::vector<int> tile_index;                  // -1 or index into tiles
     std::vector<aqs_hip::TilePass> tiles;
+    // per tile pass, the same gates with dense ops, for complex64 states (no
+    // segments where dense ops gain nothing)
+    std::vector<aqs_hip::TilePass> tiles_c64;
+    const aqs_hip::TilePass& tile(size_t i, int precision) const {
+        return precision == AQS_C64 && !tiles_c64[i].segs.empty() ? tiles_c64[i] : tiles[i];
+    }
+    // aqs_fuse_auto below 20 qubits: the tile form of the same circuit, which
+    // states run where it is modelled cheaper than the listed blocks (owned)
+    aqs_schedule_s* tile_form = nullptr;
     // device copies, built at first use for a given precision
     void* dev = nullptr;
     int dev_precision = -1;
     std::vector<size_t> dev_off;
-    std::vector<std::array<size_t, 8>> dev_tile;  // tile passes: TileDevProgram fields
+    std::vector<std::array<size_t, 9>> dev_tile;  // tile passes: TileDevProgram fields
     std::vector<char> dev_mfma;
 
     // appends a pass with no side data

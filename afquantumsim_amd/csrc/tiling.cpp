@@ -43,7 +43,15 @@ using namespace aqs_hip;
 
 namespace {
 
-constexpr int kTileAutoMinQubits = 20;
+// aqs_fuse_auto considers tiles from 10 qubits up (one tile); below 20 qubits
+// the schedule lists its blocks and keeps the tile form for its runs.  Medium
+// states take smaller tiles: more workgroups.  Measured, us for blocks, then tiles of
+// 11 / 12 / 13 qubits, random layers of depth 40: 13 qubits 296, 174 / 175 /
+// 157; 15: 343, 262 / 245 / 274; 17: 442, 374 / 364 / 389; 19: 643, 461 / 464 /
+// 490; 20: 966, 634 / 614 / 601; brickwork depth 20: 14: 148, 102 / 101 / 123;
+// 22: 926, 601 / 456 / 418.
+constexpr int kTileAutoMinQubits = 10, kTileListedMinQubits = 20;
+int auto_tile_qubits(int n) { return n <= 13 ? n : n <= 19 ? 12 : kTileMaxLocal; }
 
 // A phase term: multiply by z where every listed index bit is 1.
 struct Term {
@@ -353,8 +361,14 @@ class Tiler {
                 lp[b] = (int)tp.local.size();
                 tp.local.push_back(b);
             }
+        TilePass td;  // the same gates with dense ops
+        td.m = tp.m;
+        td.local = tp.local;
         segments(members, lp, tp);
         check_pass(tp);
+        dense_segments(members, lp, td);
+        check_pass(td);
+        if (td.dense.empty()) td = TilePass();
         for (size_t i : members) done[i] = 1;
         if (tp.segs.empty()) return;  // the gates cancelled exactly
         aqs_op op{};
@@ -362,62 +376,275 @@ class Tiler {
         sch_->push_plain(op);
         sch_->tile_index.back() = (int)sch_->tiles.size();
         sch_->tiles.push_back(std::move(tp));
+        sch_->tiles_c64.push_back(std::move(td));
     }
 
     void segments(const std::vector<size_t>& members, const std::vector<int>& lp, TilePass& tp) {
         std::vector<char> mdone(members.size(), 0);
         size_t left = members.size();
-        while (left) {
-            // slots: the first 4 distinct targets among gates that are ready
-            std::vector<int> reg;
-            std::vector<char> st(n_, 0);
-            for (size_t k = 0; k < members.size() && reg.size() < (size_t)kTileRegBits; ++k) {
-                if (mdone[k]) continue;
-                const GOp& o = g_[members[k]];
-                if (blocked(o, st)) {
-                    pass_over(o, st);
-                    continue;
-                }
-                if (o.kind == TILE_PHASES) continue;
-                const int p = lp[o.tbit];
-                if (std::find(reg.begin(), reg.end(), p) == reg.end()) reg.push_back(p);
+        while (left) register_segment(members, lp, tp, mdone, left);
+    }
+
+    // ---- dense ops ----------------------------------------------------------
+
+    // What the scan for dense blocks needs of a member: the index bits it
+    // uses, whether a dense op can hold it (no "any" controls, every bit
+    // local), and its cost in registers, in rotations.
+    struct Member {
+        uint64_t nd, dg;
+        bool fits;
+        double cost;
+    };
+
+    Member member_of(const GOp& o, const std::vector<int>& lp) const {
+        Member r{0, 0, !o.any, 0.0};
+        for (int b : o.nd) r.nd |= 1ull << b;
+        for (int b : o.dg) r.dg |= 1ull << b;
+        for (int b : o.nd) r.fits = r.fits && lp[b] >= 0;
+        for (int b : o.dg) r.fits = r.fits && lp[b] >= 0;
+        r.cost = o.kind == TILE_MAT ? 1.6 : o.kind == TILE_MATR ? 0.85 : o.kind == TILE_PHASES ? 0.3 : 1.0;
+        return r;
+    }
+
+    // Cost of the members that are ready inside the index bits `set`, in
+    // order; their numbers into `take` when given.
+    static double capture(const std::vector<Member>& ms, const std::vector<char>& mdone, uint64_t set,
+                          std::vector<size_t>* take) {
+        uint64_t nd = 0, dg = 0;
+        double c = 0;
+        for (size_t k = 0; k < ms.size() && (nd & set) != set; ++k) {
+            if (mdone[k]) continue;
+            const Member& o = ms[k];
+            if (o.fits && !((o.nd | o.dg) & ~set) && !(o.nd & (nd | dg)) && !(o.dg & nd)) {
+                c += o.cost;
+                if (take) take->push_back(k);
+            } else {
+                nd |= o.nd;
+                dg |= o.dg;
             }
-            for (int p = 0; p < m_ && reg.size() < (size_t)kTileRegBits; ++p)
-                if (std::find(reg.begin(), reg.end(), p) == reg.end()) reg.push_back(p);
-            // run every gate that is ready and fits the slots
+        }
+        return c;
+    }
+
+    // A dense op costs about 2.4 rotations of matrix-core time and as much
+    // VALU work (splitting its 32 inputs per thread), and cuts the segment.
+    // Compiled 28-qubit brickwork / 26-qubit random layers by this limit: 1.5
+    // 34.2 / 9.3 ms, 2.5 32.7 / 9.1, 3.2 31.8 / 8.9, 4.5 31.0 / 8.9 (before the
+    // split was made cheaper); 20-qubit random layers 643, 636, 626, 631 us.
+    static constexpr double kDenseMinCost = 3.2;
+
+    // The 4 local index bits whose ready members cost most, grown from the
+    // first ready members' bits (0: none worth a dense op).
+    uint64_t best_block(const std::vector<Member>& ms, const std::vector<char>& mdone, uint64_t local) const {
+        uint64_t best = 0;
+        double best_cost = kDenseMinCost;
+        uint64_t nd = 0, dg = 0, tried = 0;
+        int seeds = 0;
+        for (size_t k = 0; k < ms.size() && seeds < 3; ++k) {
+            if (mdone[k]) continue;
+            const Member& o = ms[k];
+            if ((o.nd & (nd | dg)) || (o.dg & nd) || !o.fits || !o.nd || __builtin_popcountll(o.nd | o.dg) > 4 ||
+                (o.nd & tried)) {
+                if (!(o.nd & tried)) {
+                    nd |= o.nd;
+                    dg |= o.dg;
+                }
+                continue;
+            }
+            ++seeds;
+            uint64_t set = o.nd | o.dg;
+            double c = 0;
+            while (__builtin_popcountll(set) < 4) {
+                uint64_t pick = 0;
+                double pc = -1;
+                for (uint64_t rest = local & ~set; rest; rest &= rest - 1) {
+                    const uint64_t b = rest & (0 - rest);
+                    const double bc = capture(ms, mdone, set | b, nullptr);
+                    if (bc > pc) {
+                        pc = bc;
+                        pick = b;
+                    }
+                }
+                set |= pick;
+                c = pc;
+            }
+            tried |= set;
+            if (c == 0) c = capture(ms, mdone, set, nullptr);
+            if (c > best_cost) {
+                best_cost = c;
+                best = set;
+            }
+        }
+        return best;
+    }
+
+    // Applies a member to the rows of a 16 x 16 matrix whose index bit i is
+    // index bit pos[i].
+    void dense_rows(const GOp& o, const int (&pos)[4], cd (&u)[16][16]) const {
+        auto mask_of = [&](const std::vector<int>& bits) {
+            int m = 0;
+            for (int b : bits)
+                for (int i = 0; i < 4; ++i)
+                    if (pos[i] == b) m |= 1 << i;
+            return m;
+        };
+        if (o.kind == TILE_PHASES) {
+            for (const Term& t : o.terms) {
+                const int m = mask_of(t.bits);
+                for (int r = 0; r < 16; ++r)
+                    if ((r & m) == m)
+                        for (cd& x : u[r]) x *= t.z;
+            }
+            return;
+        }
+        const int t = mask_of({o.tbit}), c = mask_of(o.ctrl);
+        for (int r = 0; r < 16; ++r) {
+            if ((r & t) || (r & c) != c) continue;
+            for (int k = 0; k < 16; ++k) {
+                cd &p = u[r][k], &q = u[r | t][k];
+                const cd p0 = p, q0 = q;
+                if (o.kind == TILE_XCH) {
+                    std::swap(p, q);
+                } else if (o.kind == TILE_MATR) {
+                    p = o.m[0] * p0 + o.m[1] * q0;
+                    q = o.m[2] * p0 + o.m[3] * q0;
+                } else if (o.kind == TILE_MATP) {
+                    q *= cd(o.m[4], o.m[5]);
+                    p -= o.m[0] * q;
+                    q += o.m[1] * p;
+                    p -= o.m[0] * q;
+                } else {
+                    p = cd(o.m[0], o.m[1]) * p0 + cd(o.m[2], o.m[3]) * q0;
+                    q = cd(o.m[4], o.m[5]) * p0 + cd(o.m[6], o.m[7]) * q0;
+                }
+            }
+        }
+    }
+
+    // The pass's gates with dense ops where they pay: a dense segment holds
+    // one dense op and then the diagonal gates that are ready and could not
+    // join one (bits outside the tile); what is left runs in register segments.
+    void dense_segments(const std::vector<size_t>& members, const std::vector<int>& lp, TilePass& tp) {
+        std::vector<char> mdone(members.size(), 0);
+        std::vector<Member> ms;
+        uint64_t local = 0;
+        for (size_t i : members) ms.push_back(member_of(g_[i], lp));
+        for (int b : tp.local) local |= 1ull << b;
+        size_t left = members.size();
+        while (left) {
+            const uint64_t set = m_ >= 10 ? best_block(ms, mdone, local) : 0;
+            if (!set) {
+                register_segment(members, lp, tp, mdone, left);
+                continue;
+            }
+            std::vector<size_t> take;
+            capture(ms, mdone, set, &take);
+            // slots 0..2 and thread bit 5: the block's bits, ascending
+            int pos[4], k = 0;
+            for (uint64_t x = set; x; x &= x - 1) pos[k++] = __builtin_ctzll(x);
             TileSegDev sd{};
+            std::vector<int> reg;
+            for (int i = 0; i < 3; ++i) reg.push_back(lp[pos[i]]);
+            const int p5 = lp[pos[3]];
+            for (int p = m_ - 1; reg.size() < (size_t)kTileRegBits; --p)
+                if (p != p5 && std::find(reg.begin(), reg.end(), p) == reg.end()) reg.push_back(p);
             for (int r = 0; r < kTileRegBits; ++r) sd.reg[r] = reg[r];
             int t = 0;
-            for (int p = 0; p < m_; ++p)
-                if (std::find(reg.begin(), reg.end(), p) == reg.end()) sd.thr[t++] = p;
+            for (int p = 0; p < m_; ++p) {
+                if (p == p5 || std::find(reg.begin(), reg.end(), p) != reg.end()) continue;
+                if (t == 5) sd.thr[t++] = p5;
+                sd.thr[t++] = p;
+            }
+            if (t == 5) sd.thr[t++] = p5;
             sd.op_begin = (uint32_t)tp.ops.size();
-            std::fill(st.begin(), st.end(), 0);
-            std::vector<const GOp*> run;  // consecutive diagonal gates, merged into one op
-            const size_t left_before = left;
-            for (size_t k = 0; k < members.size(); ++k) {
-                if (mdone[k]) continue;
-                const GOp& o = g_[members[k]];
-                const bool fits = o.kind == TILE_PHASES || std::find(reg.begin(), reg.end(), lp[o.tbit]) != reg.end();
-                if (!fits || blocked(o, st)) {
-                    pass_over(o, st);
-                    continue;
-                }
-                if (o.kind == TILE_PHASES) {
-                    run.push_back(&o);
-                } else {
-                    flush_phases(run, lp, reg, tp);
-                    push_op(o, lp, reg, tp);
-                }
-                mdone[k] = 1;
+            cd u[16][16] = {};
+            for (int r = 0; r < 16; ++r) u[r][r] = 1;
+            for (size_t i : take) {
+                dense_rows(g_[members[i]], pos, u);
+                mdone[i] = 1;
                 --left;
             }
+            TileOpDev d{};
+            d.code = kTileCodeDense;
+            d.term_begin = (uint32_t)(tp.dense.size() / kDenseDoubles);
+            tp.ops.push_back(d);
+            tp.m128.insert(tp.m128.end(), 8, 0.0);
+            for (const auto& row : u)
+                for (const cd& x : row) {
+                    tp.dense.push_back(x.real());
+                    tp.dense.push_back(x.imag());
+                }
+            std::vector<const GOp*> run;
+            uint64_t nd = 0, dg = 0;
+            for (size_t i = 0; i < ms.size(); ++i) {
+                if (mdone[i]) continue;
+                const Member& o = ms[i];
+                if (!o.nd && !o.fits && !(o.dg & nd)) {
+                    run.push_back(&g_[members[i]]);
+                    mdone[i] = 1;
+                    --left;
+                } else {
+                    nd |= o.nd;
+                    dg |= o.dg;
+                }
+            }
             flush_phases(run, lp, reg, tp);
-            group_rotations(tp, sd.op_begin);
             sd.op_count = (uint32_t)tp.ops.size() - sd.op_begin;
-            if (left == left_before) fail(AQS_ERR_RUNTIME, "tile schedule made no progress");
-            // (phase terms that multiply to exactly 1 leave nothing to run)
-            if (sd.op_count) tp.segs.push_back(sd);
+            tp.segs.push_back(sd);
         }
+    }
+
+    void register_segment(const std::vector<size_t>& members, const std::vector<int>& lp, TilePass& tp,
+                          std::vector<char>& mdone, size_t& left) {
+        // slots: the first 4 distinct targets among gates that are ready
+        std::vector<int> reg;
+        std::vector<char> st(n_, 0);
+        for (size_t k = 0; k < members.size() && reg.size() < (size_t)kTileRegBits; ++k) {
+            if (mdone[k]) continue;
+            const GOp& o = g_[members[k]];
+            if (blocked(o, st)) {
+                pass_over(o, st);
+                continue;
+            }
+            if (o.kind == TILE_PHASES) continue;
+            const int p = lp[o.tbit];
+            if (std::find(reg.begin(), reg.end(), p) == reg.end()) reg.push_back(p);
+        }
+        for (int p = 0; p < m_ && reg.size() < (size_t)kTileRegBits; ++p)
+            if (std::find(reg.begin(), reg.end(), p) == reg.end()) reg.push_back(p);
+        // run every gate that is ready and fits the slots
+        TileSegDev sd{};
+        for (int r = 0; r < kTileRegBits; ++r) sd.reg[r] = reg[r];
+        int t = 0;
+        for (int p = 0; p < m_; ++p)
+            if (std::find(reg.begin(), reg.end(), p) == reg.end()) sd.thr[t++] = p;
+        sd.op_begin = (uint32_t)tp.ops.size();
+        std::fill(st.begin(), st.end(), 0);
+        std::vector<const GOp*> run;  // consecutive diagonal gates, merged into one op
+        const size_t left_before = left;
+        for (size_t k = 0; k < members.size(); ++k) {
+            if (mdone[k]) continue;
+            const GOp& o = g_[members[k]];
+            const bool fits = o.kind == TILE_PHASES || std::find(reg.begin(), reg.end(), lp[o.tbit]) != reg.end();
+            if (!fits || blocked(o, st)) {
+                pass_over(o, st);
+                continue;
+            }
+            if (o.kind == TILE_PHASES) {
+                run.push_back(&o);
+            } else {
+                flush_phases(run, lp, reg, tp);
+                push_op(o, lp, reg, tp);
+            }
+            mdone[k] = 1;
+            --left;
+        }
+        flush_phases(run, lp, reg, tp);
+        group_rotations(tp, sd.op_begin);
+        sd.op_count = (uint32_t)tp.ops.size() - sd.op_begin;
+        if (left == left_before) fail(AQS_ERR_RUNTIME, "tile schedule made no progress");
+        // (phase terms that multiply to exactly 1 leave nothing to run)
+        if (sd.op_count) tp.segs.push_back(sd);
     }
 
     // Every position the kernel turns into an LDS address or shift stays in
@@ -440,7 +667,7 @@ class Tiler {
             // the mask's other slots, ascending
             for (uint32_t o = s.op_begin; ok && o < s.op_begin + s.op_count; ++o) {
                 const int code = tp.ops[o].code;
-                if (code < kTileCodeMatPSet || code >= kTileCodeCount) continue;
+                if (code < kTileCodeMatPSet || code >= kTileCodeDense) continue;
                 const uint32_t mask = (uint32_t)(code - kTileCodeMatPSet);
                 const uint32_t pc = (uint32_t)__builtin_popcount(mask);
                 ok = pc >= 2 && o + pc <= s.op_begin + s.op_count;
@@ -449,7 +676,12 @@ class Tiler {
                     ok = tp.ops[o + k].code == kTileCodeMatP + __builtin_ctz(rest);
             }
         }
+        ok = ok && tp.dense.size() % kDenseDoubles == 0;
         for (const auto& o : tp.ops) {
+            if (o.code == kTileCodeDense) {
+                ok = ok && (size_t)o.term_begin < tp.dense.size() / kDenseDoubles;
+                continue;
+            }
             ok = ok && o.code >= 0 && o.code < kTileCodeCount && o.c_reg < (1u << kTileRegBits) &&
                  o.c_thr < (1u << m) && (o.c_glb >> n_) == 0;
             if (!tile_code_is_phases(o.code)) {
@@ -682,7 +914,7 @@ class Tiler {
 // 0.053 of a sweep, a real 2x2 0.05, an exchange 0.066, a phase term 0.02
 // and each product a phase run applies per thread 0.0045; a complex 2x2,
 // absent from those circuits, is priced at 0.085 (16 multiply-adds per
-// pair against a rotation's 10).  Other passes (fitted earlier at 22..28
+// pair against a rotation's 10); a dense op takes 0.15 with its LDS round trip.  Other passes (fitted earlier at 22..28
 // qubits, mean error 9%): an MFMA block 1.17-1.2, a
 // diagonal table 1.25 (0.05 when it rides in a neighbouring MFMA block), a
 // bit permutation 1.8, a plain one-qubit pass 1, a sparse pass its touched
@@ -690,10 +922,12 @@ class Tiler {
 double pass_cost(const aqs_schedule_s* sch, size_t p) {
     const aqs_op& op = sch->passes[p];
     if (sch->tile_index[p] >= 0) {
-        const TilePass& t = sch->tiles[sch->tile_index[p]];
+        const TilePass& t = sch->tile(sch->tile_index[p], AQS_C64);
         double c = 1.03;
         for (const auto& o : t.ops) {
-            if (o.code < 12) {
+            if (o.code == kTileCodeDense) {
+                c += 0.15;
+            } else if (o.code < 12) {
                 c += 0.085;
             } else if (o.code >= kTileCodeMatP) {
                 c += 0.053;
@@ -769,6 +1003,43 @@ bool diag_rides_block(const aqs_schedule_s* sch, size_t p) {
 
 }  // namespace
 
+// Operand A of v_mfma_f32_32x32x16_bf16 for each unitary, [plane][real or
+// imaginary columns][lane][8]: lane l holds row l % 32, columns 8 (l / 32) + j
+// of the real form.  Row 8 g + 4 h + e is part g % 2 of amplitude
+// 8 h + 4 (g / 2) + e.
+std::vector<uint16_t> aqs_hip::pack_dense(const std::vector<double>& dense) {
+    const size_t count = dense.size() / kDenseDoubles;
+    std::vector<uint16_t> out(count * kDenseOperand);
+    auto bf16 = [](double v, double& back) {  // to nearest, ties to even
+        const float f = (float)v;
+        uint32_t w;
+        std::memcpy(&w, &f, 4);
+        w += 0x7FFFu + ((w >> 16) & 1u);
+        w &= 0xFFFF0000u;
+        float r;
+        std::memcpy(&r, &w, 4);
+        back = r;
+        return (uint16_t)(w >> 16);
+    };
+    for (size_t c = 0; c < count; ++c) {
+        const double* u = dense.data() + c * kDenseDoubles;
+        for (int s = 0; s < 2; ++s)
+            for (int l = 0; l < 64; ++l)
+                for (int j = 0; j < 8; ++j) {
+                    const int row = l % 32, g = row / 8, h = (row / 4) % 2, e = row % 4;
+                    const int amp = 8 * h + 4 * (g / 2) + e, col = 8 * (l / 32) + j;
+                    const double re = u[2 * (16 * amp + col)], im = u[2 * (16 * amp + col) + 1];
+                    double v = g % 2 == 0 ? (s == 0 ? re : -im) : (s == 0 ? im : re);
+                    for (int p = 0; p < 3; ++p) {
+                        double back;
+                        out[c * kDenseOperand + (size_t)(((2 * p + s) * 64 + l) * 8 + j)] = bf16(v, back);
+                        v -= back;
+                    }
+                }
+    }
+    return out;
+}
+
 double aqs_hip::schedule_cost(const aqs_schedule_s* sch) {
     double c = 0;
     for (size_t p = 0; p < sch->passes.size(); ++p)
@@ -819,10 +1090,6 @@ aqs_status aqs_fuse_auto(const aqs_op* ops, size_t count, int nqubits, aqs_sched
     }
     *out = nullptr;
     aqs_schedule blocks = nullptr, tiled = nullptr;
-    // below 2^20 amplitudes the state stays in the caches and launches of
-    // the block schedule are cheaper than in-tile work (measured: at 19
-    // qubits blocks win, at 20-21 tiles by 5-40% on brickwork and random
-    // layers)
     if (nqubits < kTileAutoMinQubits) return aqs_fuse(ops, count, nqubits, 5, out);
     // both schedules, the tile one on a thread of its own (its error
     // message, kept per thread, is carried back)
@@ -831,7 +1098,7 @@ aqs_status aqs_fuse_auto(const aqs_op* ops, size_t count, int nqubits, aqs_sched
     std::thread worker;
     bool threaded = false;
     auto fuse_tiles = [&] {
-        tst = aqs_fuse_tiled(ops, count, nqubits, 0, &tiled);
+        tst = aqs_fuse_tiled(ops, count, nqubits, auto_tile_qubits(nqubits), &tiled);
         if (tst != AQS_OK) terr = aqs_last_error();
     };
     try {
@@ -853,6 +1120,11 @@ aqs_status aqs_fuse_auto(const aqs_op* ops, size_t count, int nqubits, aqs_sched
         return tst;
     }
     const bool keep_tiled = schedule_cost(tiled) < schedule_cost(blocks);
+    if (keep_tiled && nqubits < kTileListedMinQubits) {
+        blocks->tile_form = tiled;
+        *out = blocks;
+        return AQS_OK;
+    }
     aqs_schedule_destroy(keep_tiled ? blocks : tiled);
     *out = keep_tiled ? tiled : blocks;
     return AQS_OK;

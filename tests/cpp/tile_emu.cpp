@@ -166,19 +166,45 @@ void tile_apply(std::vector<cplx>& v, int n, const TilePass& tp) {
                 if ((base & tp.fold_terms[e].m_glb) == tp.fold_terms[e].m_glb)
                     fold_val[f] *= cplx(tp.fold_z128[2 * e], tp.fold_z128[2 * e + 1]);
         for (const auto& S : tp.segs) {
-            for (uint32_t tid = 0; tid < (1u << W); ++tid) {
-                uint32_t lthr = 0;
-                for (int b = 0; b < W; ++b) lthr |= ((tid >> b) & 1u) << S.thr[b];
-                auto addr = [&](int j) {
-                    uint32_t l = lthr;
-                    for (int r = 0; r < kTileRegBits; ++r)
-                        if ((j >> r) & 1) l |= 1u << S.reg[r];
-                    return l;
-                };
-                cplx x[16];
-                for (int j = 0; j < 16; ++j) x[j] = tile[addr(j)];
-                for (uint32_t o = 0; o < S.op_count; ++o) {
-                    const TileOpDev& op = tp.ops[S.op_begin + o];
+            auto thr_bits = [&](uint32_t tid) {
+                uint32_t l = 0;
+                for (int b = 0; b < W; ++b) l |= ((tid >> b) & 1u) << S.thr[b];
+                return l;
+            };
+            auto addr = [&](uint32_t lthr, int j) {
+                uint32_t l = lthr;
+                for (int r = 0; r < kTileRegBits; ++r)
+                    if ((j >> r) & 1) l |= 1u << S.reg[r];
+                return l;
+            };
+            for (uint32_t o = 0; o < S.op_count; ++o) {
+                const TileOpDev& op = tp.ops[S.op_begin + o];
+                if (op.code == kTileCodeDense) {
+                    // block index bits 0..2: slots 0..2, bit 3: thread bit 5;
+                    // slot 3 and the other thread bits: columns
+                    const double* u = tp.dense.data() + op.term_begin * kDenseDoubles;
+                    for (uint32_t tid = 0; tid < (1u << W); ++tid) {
+                        if (tid & 32u) continue;
+                        for (int q = 0; q < 2; ++q) {
+                            cplx in[16], out[16];
+                            for (int r = 0; r < 16; ++r)
+                                in[r] = tile[addr(thr_bits(tid | (r & 8 ? 32u : 0u)), 8 * q + (r & 7))];
+                            for (int r = 0; r < 16; ++r)
+                                for (int c = 0; c < 16; ++c)
+                                    out[r] += cplx(u[2 * (16 * r + c)], u[2 * (16 * r + c) + 1]) * in[c];
+                            for (int r = 0; r < 16; ++r)
+                                tile[addr(thr_bits(tid | (r & 8 ? 32u : 0u)), 8 * q + (r & 7))] = out[r];
+                        }
+                    }
+                    continue;
+                }
+                for (uint32_t tid = 0; tid < (1u << W); ++tid) {
+                    const uint32_t lthr = thr_bits(tid);
+                    cplx x[16];
+                    for (int j = 0; j < 16; ++j) x[j] = tile[addr(lthr, j)];
+                    auto store = [&] {
+                        for (int j = 0; j < 16; ++j) tile[addr(lthr, j)] = x[j];
+                    };
                     if (tile_code_is_phases(op.code)) {
                         // every term multiplies the amplitudes whose register
                         // index holds its register mask (both device forms
@@ -191,6 +217,7 @@ void tile_apply(std::vector<cplx>& v, int n, const TilePass& tp) {
                             for (int j = 0; j < 16; ++j)
                                 if (((uint32_t)j & t.m_reg) == t.m_reg) x[j] *= z;
                         }
+                        store();
                         continue;
                     }
                     const bool any = op.any != 0;
@@ -236,8 +263,8 @@ void tile_apply(std::vector<cplx>& v, int n, const TilePass& tp) {
                             std::swap(x[j], x[k]);
                         }
                     }
+                    store();
                 }
-                for (int j = 0; j < 16; ++j) tile[addr(j)] = x[j];
             }
         }
         for (uint32_t l = 0; l < tile.size(); ++l) v[gidx(l)] = tile[l];
@@ -348,17 +375,19 @@ extern "C" {
 // Builds the tiled schedule of ops and applies it to `state` (2^n complex
 // FP64, interleaved) on the host.  Returns the aqs_status of the build;
 // counts[0..3] = passes, tile passes, segments, folded term groups.
-int tile_emulate(const aqs_op* ops, size_t count, int n, int tile_qubits, double* state, size_t* counts) {
+static int tile_emulate_as(const aqs_op* ops, size_t count, int n, int tile_qubits, int precision, double* state,
+                           size_t* counts) {
     aqs_schedule sch = nullptr;
     const int st = aqs_fuse_tiled(ops, count, n, tile_qubits, &sch);
     if (st != AQS_OK) return st;
     std::vector<cplx> v((size_t)1 << n);
     std::memcpy(v.data(), state, v.size() * sizeof(cplx));
-    size_t tiles = 0, segs = 0, folds = 0;
+    size_t tiles = 0, segs = 0, folds = 0, dense = 0;
     for (size_t p = 0; p < sch->passes.size(); ++p) {
         const aqs_op& op = sch->passes[p];
         if (sch->tile_index[p] >= 0) {
-            const TilePass& tp = sch->tiles[sch->tile_index[p]];
+            const TilePass& tp = sch->tile(sch->tile_index[p], precision);
+            dense += tp.dense.size() / kDenseDoubles;
             try {
                 tile_apply(v, n, tp);
             } catch (int) {
@@ -382,9 +411,19 @@ int tile_emulate(const aqs_op* ops, size_t count, int n, int tile_qubits, double
     counts[0] = sch->passes.size();
     counts[1] = tiles;
     counts[2] = segs;
-    counts[3] = folds;
+    counts[3] = precision == AQS_C64 ? dense : folds;
     aqs_schedule_destroy(sch);
     return AQS_OK;
+}
+
+int tile_emulate(const aqs_op* ops, size_t count, int n, int tile_qubits, double* state, size_t* counts) {
+    return tile_emulate_as(ops, count, n, tile_qubits, AQS_C128, state, counts);
+}
+
+// The programs that complex64 states run (dense ops, their unitaries in
+// FP64).  counts[3] = dense ops.
+int tile_emulate_c64(const aqs_op* ops, size_t count, int n, int tile_qubits, double* state, size_t* counts) {
+    return tile_emulate_as(ops, count, n, tile_qubits, AQS_C64, state, counts);
 }
 
 // Builds the dense-block schedule of ops (aqs_fuse, blocks of at most kmax

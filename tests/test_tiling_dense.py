@@ -1,0 +1,65 @@
+"""Dense ops of tile passes (complex64 programs): runs of gates on 4 local
+positions as one 16 x 16 unitary.  The emulation (tests/cpp/tile_emu.cpp,
+tile_emulate_c64) reads the programs that complex64 states run with their
+unitaries in FP64: 1e-12 against the oracle; on the GPU the matrix-core
+products against the complex128 path."""
+import ctypes
+
+import numpy as np
+import pytest
+
+import oracle
+from afquantumsim_amd import circuits, hip, ops
+from tests.helpers import random_state
+from tests.test_tiling import emu, random_all_kinds  # noqa: F401
+
+
+def emulate_c64(lib, n, sv, lowered, tile_qubits=0):
+    f = lib.tile_emulate_c64
+    f.restype = ctypes.c_int
+    f.argtypes = lib.tile_emulate.argtypes
+    p = hip.PackedOps(lowered)
+    v = np.ascontiguousarray(sv, dtype=np.complex128).copy()
+    counts = (ctypes.c_size_t * 4)()
+    rc = f(p.arr, p.count, n, tile_qubits, v.ctypes.data, counts)
+    assert rc == 0, (rc, hip.load().aqs_last_error())
+    return v, tuple(counts)
+
+
+@pytest.mark.parametrize("name", ["brickwork", "layers", "ansatz", "qft", "kinds"])
+@pytest.mark.parametrize("n,tile", [(10, 10), (11, 0), (13, 0), (14, 11), (15, 13)])
+def test_dense_programs(emu, name, n, tile):  # noqa: F811
+    gates = {"brickwork": lambda: circuits.brickwork(n, 8, seed=n), "layers": lambda: circuits.random_layered(n, 8, seed=n),
+             "ansatz": lambda: circuits.ry_rz_ladder(n, 5, np.random.default_rng(n)),
+             "qft": lambda: circuits.fourier_transform(n), "kinds": lambda: random_all_kinds(n, 150, n)}[name]()
+    sv = random_state(n, 4)
+    got, counts = emulate_c64(emu, n, sv, ops.lower_all(gates, exact=True), tile)
+    np.testing.assert_allclose(got, oracle.run(sv, n, gates, threads=8), atol=1e-12, rtol=0)
+    if name in ("brickwork", "layers"):
+        assert counts[3] > 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tile", [10, 11, 12, 13])
+@pytest.mark.parametrize("scale", [1.0, 1e-20, 1e15])
+def test_dense_products_keep_fp32_accuracy(tile, scale):
+    """Brickwork of depth 12 at every tile size, on states of any scale (bf16
+    has FP32's range): each of the at most 12 x 14 gates and blocks rounds like
+    FP32, 2^-24 of the norm, independent in sign: sqrt(168) 6e-8 = 8e-7; four
+    times that allowed."""
+    hip.init(0)
+    n = 14
+    gates = circuits.brickwork(n, 12, seed=tile)
+    sv = (random_state(n, 3) * scale).astype(np.complex64)
+    sch = hip.Schedule(ops.lower_all(gates), n, mode="tiled", tile_qubits=tile)
+    st = hip.State(n, hip.C64)
+    st.upload(sv)
+    st.apply_schedule(sch)
+    got = st.download().astype(np.complex128)
+    ref = hip.State(n, hip.C128)
+    ref.upload(sv.astype(np.complex128))
+    ref.apply(ops.lower_all(gates, exact=True))
+    want = ref.download()
+    for x in (st, ref):
+        x.close()
+    assert np.linalg.norm(got - want) < 3.2e-6 * np.linalg.norm(want)

@@ -515,6 +515,30 @@ def test_prob1_all_sizes(n, precision):
 
 
 @pytest.mark.parametrize("precision", [hip.C64, hip.C128], ids=["c64", "c128"])
+@pytest.mark.parametrize("n", [3, 9, 14])
+def test_measure_every_qubit(n, precision):
+    """P(1) reads half of the state where the qubit's runs fill 64 bytes and
+    all of it below; a collapse writes the dropped half without reading it.
+    Every qubit, both outcomes: FP64 probabilities to 1e-13, amplitudes to the
+    rounding of one scaling."""
+    st = hip.State(n, precision)
+    for q in range(n):
+        for u in (0.02, 0.98):
+            st.gaussian(17 + q)
+            sv = st.download().astype(np.complex128)
+            ones = ((np.arange(1 << n) >> (n - 1 - q)) & 1) == 1
+            p1 = (np.abs(sv[ones]) ** 2).sum()
+            outcome, got = st.measure_qubit(q, u)
+            assert abs(got - p1) < 1e-13 and outcome == int(u < p1)
+            keep = ones == bool(outcome)
+            want = np.where(keep, sv / np.sqrt(p1 if outcome else 1 - p1), 0)
+            out = st.download()
+            np.testing.assert_allclose(out, want, rtol=0, atol=2e-7 if precision == hip.C64 else 1e-13)
+            assert not out[~keep].any()
+    st.close()
+
+
+@pytest.mark.parametrize("precision", [hip.C64, hip.C128], ids=["c64", "c128"])
 def test_measure_qubit_collapse(precision):
     """Qubit n-1 (bit 0) splits each 16-byte pair of complex64 amplitudes
     between kept and zeroed; the zeroed ones are exactly +0."""

@@ -263,9 +263,10 @@ static int run_tile_qubits(int n, int precision) {
     return n <= 11 ? n : n <= 18 ? 11 : kRunMaxTileC128;
 }
 
-void apply_run(aqs_state s, const aqs_op* ops, size_t count) {
+size_t apply_run(aqs_state s, const aqs_op* ops, size_t count) {
     const int m = run_tile_qubits(s->n, s->precision);
-    for (const RunLaunch& l : plan_runs(ops, count, s->n, m, s->precision)) {
+    const std::vector<RunLaunch> launches = plan_runs(ops, count, s->n, m, s->precision);
+    for (const RunLaunch& l : launches) {
         RunArgs a;
         a.sv = s->amps;
         a.n = (uint32_t)s->n;
@@ -280,6 +281,7 @@ void apply_run(aqs_state s, const aqs_op* ops, size_t count) {
         else
             launch_run<double2, double>(s, a);
     }
+    return launches.size();
 }
 
 }  // namespace aqs_hip

@@ -997,10 +997,12 @@ aqs_batch check_batch(aqs_batch b) {
 
 namespace aqs_hip {
 
+static_assert(kGroupMaxQubits <= kGroupSampleQubits, "group members are sampled as small states");
+
 namespace {
 
 constexpr size_t kArenaAlign = 256;
-constexpr int kGroupRegions = 9;  // aligned regions of the arena layout
+constexpr int kGroupRegions = 10;  // aligned regions of the arena layout
 
 size_t align_up(size_t x) { return (x + kArenaAlign - 1) / kArenaAlign * kArenaAlign; }
 
@@ -1014,8 +1016,8 @@ size_t group_item_bytes(int n, size_t nops, uint32_t shots) {
     const size_t items = n > kGroupLdsQubits ? (nops + 1) * tiles : 1;
     const size_t prog = sizeof(Desc) + items * sizeof(BatchItem) + (nops + 1) * sizeof(BatchPhase) +
                         3 * nops * sizeof(BatchSeg) + 3 * nops * sizeof(BatchOp);
-    const size_t io = sizeof(double) + 2 * sizeof(uint64_t) * (size_t)shots;  // norm, u, indices
-    return prog + io + align_up(sizeof(float2) << n) + align_up(sample_norm_scratch_bytes(n)) +
+    const size_t io = sizeof(SampleItem) + sizeof(double) + 2 * sizeof(uint64_t) * (size_t)shots;  // norm, u, indices
+    return prog + io + align_up(sizeof(float2) << n) + align_up(sample_group_table_bytes(n)) +
            kGroupRegions * kArenaAlign;
 }
 
@@ -1043,7 +1045,7 @@ void run_group(GroupItem* items, int count, void* arena, size_t arena_bytes, hip
         shot_off[k] = shots_total;
         shots_total += items[k].shots;
     }
-    // arena layout: upload (desc, items, phases, segs, ops, u) | download
+    // arena layout: upload (desc, items, phases, segs, ops, u, samples) | download
     // (norms, indices) | states | sampling scratch
     size_t off = 0;
     auto take = [&](size_t bytes) {
@@ -1068,17 +1070,18 @@ void run_group(GroupItem* items, int count, void* arena, size_t arena_bytes, hip
     const size_t o_segs = take(sizeof(BatchSeg) * std::max<size_t>(1, segs.size()));
     const size_t o_ops = take(sizeof(BatchOp) * std::max<size_t>(1, ops.size()));
     const size_t o_u = take(sizeof(double) * std::max<size_t>(1, shots_total));
+    const size_t o_smp = take(sizeof(SampleItem) * count);
     const size_t o_norm = take(sizeof(double) * count);
     const size_t o_idx = take(sizeof(uint64_t) * std::max<size_t>(1, shots_total));
     std::vector<size_t> o_state(count), o_scr(count);
     for (int k = 0; k < count; ++k) o_state[k] = take(sizeof(float2) << items[k].n);
-    for (int k = 0; k < count; ++k) o_scr[k] = take(sample_norm_scratch_bytes(items[k].n));
+    for (int k = 0; k < count; ++k) o_scr[k] = take(sample_group_table_bytes(items[k].n));
     if (off > arena_bytes) fail(AQS_ERR_RUNTIME, "request group exceeds its device arena");
     char* base = (char*)arena;
     // amplitude offsets from the first state (the kernel's pool)
     for (Desc& d : desc) d.amp_offset = (o_state[d.index] - o_state[0]) / sizeof(float2);
 
-    // one upload: desc .. u are contiguous
+    // one upload: desc .. the sampling items are contiguous
     std::vector<char> up(o_norm - o_desc);
     std::memcpy(up.data(), desc.data(), sizeof(Desc) * desc.size());
     std::memcpy(up.data() + (o_items - o_desc), levels.items.data(), sizeof(BatchItem) * levels.items.size());
@@ -1089,6 +1092,18 @@ void run_group(GroupItem* items, int count, void* arena, size_t arena_bytes, hip
         if (items[k].shots)
             std::memcpy(up.data() + (o_u - o_desc) + sizeof(double) * shot_off[k], items[k].u,
                         sizeof(double) * items[k].shots);
+    uint32_t max_shots = 0;
+    for (int k = 0; k < count; ++k) {
+        const SampleItem s{base + o_state[k],
+                           (uint64_t*)(base + o_scr[k]),
+                           (const double*)(base + o_u) + shot_off[k],
+                           (uint64_t*)(base + o_idx) + shot_off[k],
+                           (double*)(base + o_norm) + k,
+                           (uint32_t)items[k].n,
+                           items[k].shots};
+        std::memcpy(up.data() + (o_smp - o_desc) + sizeof(SampleItem) * k, &s, sizeof(s));
+        max_shots = std::max(max_shots, s.shots);
+    }
     AQS_HIP(hipMemcpyAsync(base + o_desc, up.data(), up.size(), hipMemcpyHostToDevice, stream));
 
     set_lds_limit();
@@ -1096,10 +1111,7 @@ void run_group(GroupItem* items, int count, void* arena, size_t arena_bytes, hip
                   (const BatchPhase*)(base + o_phases), (const BatchSeg*)(base + o_segs),
                   (const BatchOp*)(base + o_ops), (float2*)(base + o_state[0]), nullptr, kGroupBlock, kGroupLdsQubits,
                   stream);
-    for (int k = 0; k < count; ++k)
-        queue_sample_norm(base + o_state[k], items[k].n, base + o_scr[k],
-                          (const double*)(base + o_u) + shot_off[k], items[k].shots,
-                          (uint64_t*)(base + o_idx) + shot_off[k], (double*)(base + o_norm) + k, stream);
+    queue_sample_group((const SampleItem*)(base + o_smp), count, max_shots, stream);
     std::vector<char> down(o_state[0] - o_norm);
     AQS_HIP(hipMemcpyAsync(down.data(), base + o_norm, down.size(), hipMemcpyDeviceToHost, stream));
     for (int k = 0; k < count; ++k)

@@ -167,15 +167,22 @@ void validate_op(const aqs_op& op, int nqubits);
 double reduce_norm2(aqs_state s);
 void scale_state(aqs_state s, double factor);
 
-// Device bytes that queue_sample_norm needs as scratch for a complex64 state
-// of 2^n amplitudes (sampling tables and reduction partials).
-size_t sample_norm_scratch_bytes(int n);
-// Queues on `stream`, without waiting: `shots` indices sampled from the
-// complex64 state `amps` of 2^n amplitudes (uniforms du and indices dout on
-// the device; the exact fixed-point CDF of aqs_sample) and its FP64 norm^2
-// into *dnorm (device).
-void queue_sample_norm(const void* amps, int n, void* scratch, const double* du, uint32_t shots, uint64_t* dout,
-                       double* dnorm, hipStream_t stream);
+// Norm and samples of a group of small complex64 states (at most
+// kGroupSampleQubits qubits each), queued without waiting as two launches for
+// the whole group: `shots` indices of each state by the exact fixed-point CDF
+// of aqs_sample and its FP64 norm^2.  `items` is the device copy of
+// the array; a state's `tables` hold sample_group_table_bytes(n).
+constexpr int kGroupSampleQubits = 16;
+struct SampleItem {
+    const void* amps;    // 2^n complex64 amplitudes
+    uint64_t* tables;
+    const double* u;     // shots uniforms
+    uint64_t* out;       // shots indices
+    double* norm;
+    uint32_t n, shots;
+};
+size_t sample_group_table_bytes(int n);
+void queue_sample_group(const SampleItem* items, int count, uint32_t max_shots, hipStream_t stream);
 
 // Streaming (non-temporal) 8- and 16-byte accesses: a gate pass touches each
 // amplitude once, so the lines are not kept in the caches.

@@ -377,14 +377,14 @@ __global__ __launch_bounds__(kBlock) void k_probs(const T2* __restrict__ a, uint
 // integer sum and last non-zero index, with no LDS and no barrier (exact in
 // any order).  (A 256-thread workgroup per block with LDS trees read a
 // 30-qubit complex64 state at 4.9 TB/s.)
+// Block b by this wavefront: the sum and last non-zero index in every lane,
+// and this lane's part of the FP64 sum of |a|^2.
 template <typename T2>
-__global__ __launch_bounds__(kBlock) void k_block_sums(const T2* __restrict__ a, uint64_t N, uint64_t nb,
-                                                       uint64_t* __restrict__ sums, int64_t* __restrict__ lastnz) {
+__device__ __forceinline__ double block_sum(const T2* __restrict__ a, uint64_t N, uint64_t b, uint64_t& sum,
+                                            int64_t& lastnz) {
     constexpr int A = sizeof(T2) == 8 ? 2 : 1;       // amplitudes per 16-byte unit
     constexpr int UPB = kSampleBlock / A;            // units per block
     constexpr int UPL = UPB / 64;                    // units per lane
-    const uint64_t b = (uint64_t)blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6);
-    if (b >= nb) return;
     const int lane = threadIdx.x & 63;
     const float4* av = reinterpret_cast<const float4*>(a);
     const uint64_t NV = N / A;
@@ -396,27 +396,43 @@ __global__ __launch_bounds__(kBlock) void k_block_sums(const T2* __restrict__ a,
     }
     uint64_t acc = 0;
     int64_t last = -1;
+    double p = 0.0;
 #pragma unroll
     for (int j = 0; j < UPL; ++j) {
         const uint64_t k = b * UPB + (uint64_t)j * 64 + lane;
         if (A == 2) {
-            const uint64_t q0 = quantise(prob_of(make_float2(v[j].x, v[j].y)));
-            const uint64_t q1 = quantise(prob_of(make_float2(v[j].z, v[j].w)));
+            const double p0 = prob_of(make_float2(v[j].x, v[j].y)), p1 = prob_of(make_float2(v[j].z, v[j].w));
+            const uint64_t q0 = quantise(p0);
+            const uint64_t q1 = quantise(p1);
+            p += p0 + p1;
             acc += q0 + q1;
             if (q0) last = max(last, (int64_t)(2 * k));
             if (q1) last = max(last, (int64_t)(2 * k + 1));
         } else {
             double2 d;
             __builtin_memcpy(&d, &v[j], sizeof(d));
-            const uint64_t q = quantise(prob_of(d));
+            const double p0 = prob_of(d);
+            const uint64_t q = quantise(p0);
             acc += q;
+            p += p0;
             if (q) last = max(last, (int64_t)k);
         }
     }
-    acc = wave_sum(acc);
-    last = wave_max(last);
-    if (lane == 0) {
-        sums[b] = acc;
+    sum = wave_sum(acc);
+    lastnz = wave_max(last);
+    return p;
+}
+
+template <typename T2>
+__global__ __launch_bounds__(kBlock) void k_block_sums(const T2* __restrict__ a, uint64_t N, uint64_t nb,
+                                                       uint64_t* __restrict__ sums, int64_t* __restrict__ lastnz) {
+    const uint64_t b = (uint64_t)blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6);
+    if (b >= nb) return;
+    uint64_t sum;
+    int64_t last;
+    (void)block_sum(a, N, b, sum, last);
+    if ((threadIdx.x & 63) == 0) {
+        sums[b] = sum;
         lastnz[b] = last;
     }
 }
@@ -499,15 +515,13 @@ __global__ __launch_bounds__(kBlock) void k_scan_fixup(uint64_t* __restrict__ in
     if (b < nb) incl[b] += cexcl[b / kScanChunk];
 }
 
-// One wavefront per shot.
+// One shot by this wavefront.
 template <typename T2>
-__global__ __launch_bounds__(kBlock) void k_sample(const T2* __restrict__ a, uint64_t N, const uint64_t* __restrict__ sums,
-                                                   const uint64_t* __restrict__ incl, const uint64_t* __restrict__ misc,
-                                                   uint64_t nb, const double* __restrict__ u, uint32_t shots,
-                                                   uint64_t* __restrict__ out) {
+__device__ __forceinline__ void sample_shot(const T2* __restrict__ a, uint64_t N, const uint64_t* __restrict__ sums,
+                                            const uint64_t* __restrict__ incl, const uint64_t* __restrict__ misc,
+                                            uint64_t nb, const double* __restrict__ u, uint32_t shot,
+                                            uint64_t* __restrict__ out) {
     const int lane = threadIdx.x & 63;
-    const uint32_t shot = blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6);
-    if (shot >= shots) return;
     const uint64_t thr = (uint64_t)floor(u[shot] * kFixScale);
     const uint64_t total = misc[0];
     if (thr >= total) {
@@ -559,6 +573,77 @@ __global__ __launch_bounds__(kBlock) void k_sample(const T2* __restrict__ a, uin
         }
         out[shot] = idx;
     }
+}
+
+// One wavefront per shot.
+template <typename T2>
+__global__ __launch_bounds__(kBlock) void k_sample(const T2* __restrict__ a, uint64_t N, const uint64_t* __restrict__ sums,
+                                                   const uint64_t* __restrict__ incl, const uint64_t* __restrict__ misc,
+                                                   uint64_t nb, const double* __restrict__ u, uint32_t shots,
+                                                   uint64_t* __restrict__ out) {
+    const uint32_t shot = blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6);
+    if (shot < shots) sample_shot(a, N, sums, incl, misc, nb, u, shot, out);
+}
+
+// ---- a group of small states ------------------------------------------------
+// One workgroup of 16 waves per state makes its tables (at most 64 blocks, so
+// one wave scans them) and its norm in one read; one launch then takes every
+// state's shots.  Member by member this was seven launches per state, 4 us
+// each: more than the states' gates for a group of 24.
+constexpr int kGroupWaves = 16;
+constexpr int kGroupBlocks = (1 << kGroupSampleQubits) / kSampleBlock;
+static_assert(kGroupBlocks == 64, "one wave scans a member's blocks");
+
+__global__ __launch_bounds__(64 * kGroupWaves) void k_group_tables(const SampleItem* __restrict__ items) {
+    __shared__ uint64_t s_sum[kGroupBlocks];
+    __shared__ int64_t s_last[kGroupBlocks];
+    __shared__ double s_norm[kGroupWaves];
+    const SampleItem it = items[blockIdx.x];
+    const uint64_t N = 1ull << it.n, nb = (N + kSampleBlock - 1) / kSampleBlock;
+    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    double p = 0.0;
+    for (uint64_t b = w; b < kGroupBlocks; b += kGroupWaves) {
+        uint64_t sum = 0;
+        int64_t last = -1;
+        if (b < nb) p += block_sum((const float2*)it.amps, N, b, sum, last);
+        if (lane == 0) {
+            s_sum[b] = sum;
+            s_last[b] = last;
+        }
+    }
+    p = wave_sum(p);
+    if (lane == 0) s_norm[w] = p;
+    __syncthreads();
+    if (w != 0) return;
+    const uint64_t own = s_sum[lane];
+    uint64_t incl = own;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const uint64_t v = (uint64_t)__shfl_up((unsigned long long)incl, o);
+        if (lane >= o) incl += v;
+    }
+    const int64_t last = wave_max(s_last[lane]);
+    if ((uint64_t)lane < nb) {
+        it.tables[lane] = own;
+        it.tables[nb + lane] = incl;
+    }
+    if (lane == 63) {
+        it.tables[2 * nb] = incl;
+        it.tables[2 * nb + 1] = (uint64_t)last;
+    }
+    if (lane == 0) {
+        double s = 0.0;
+        for (int k = 0; k < kGroupWaves; ++k) s += s_norm[k];
+        *it.norm = s;
+    }
+}
+
+__global__ __launch_bounds__(kBlock) void k_group_sample(const SampleItem* __restrict__ items) {
+    const SampleItem it = items[blockIdx.y];
+    const uint32_t shot = blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6);
+    if (shot >= it.shots) return;
+    const uint64_t N = 1ull << it.n, nb = (N + kSampleBlock - 1) / kSampleBlock;
+    sample_shot((const float2*)it.amps, N, it.tables, it.tables + nb, it.tables + 2 * nb, nb, it.u, shot, it.out);
 }
 
 unsigned red_grid(uint64_t N) {
@@ -687,23 +772,17 @@ namespace aqs_hip {
 
 double reduce_norm2(aqs_state s) { return reduce_mode<0>(s, 0); }
 
-size_t sample_norm_scratch_bytes(int n) {
-    const uint64_t N = 1ull << n;
-    const uint64_t nb = (N + kSampleBlock - 1) / kSampleBlock;
-    return sample_table_bytes(nb) + sizeof(double) * red_grid(N);
+size_t sample_group_table_bytes(int n) {
+    const uint64_t nb = ((1ull << n) + kSampleBlock - 1) / kSampleBlock;
+    return (size_t)(2 * nb + 2) * sizeof(uint64_t);
 }
 
-void queue_sample_norm(const void* amps, int n, void* scratch, const double* du, uint32_t shots, uint64_t* dout,
-                       double* dnorm, hipStream_t stream) {
-    const uint64_t N = 1ull << n;
-    const uint64_t nb = (N + kSampleBlock - 1) / kSampleBlock;
-    double* partial = (double*)((char*)scratch + sample_table_bytes(nb));
-    const unsigned g = red_grid(N);
-    hipLaunchKernelGGL((k_reduce<float2, 0>), dim3(g), dim3(kBlock), 0, stream, (const float2*)amps,
-                       N / 2, -1, 0ull, n, partial);
-    hipLaunchKernelGGL(k_reduce_final, dim3(1), dim3(kBlock), 0, stream, (const double*)partial, (int)g, 1, dnorm);
+void queue_sample_group(const SampleItem* items, int count, uint32_t max_shots, hipStream_t stream) {
+    hipLaunchKernelGGL(k_group_tables, dim3((unsigned)count), dim3(64 * kGroupWaves), 0, stream, items);
+    if (max_shots)
+        hipLaunchKernelGGL(k_group_sample, dim3((max_shots + kBlock / 64 - 1) / (kBlock / 64), (unsigned)count),
+                           dim3(kBlock), 0, stream, items);
     AQS_HIP(hipGetLastError());
-    if (shots) launch_sampling(amps, AQS_C64, N, sample_tables(scratch, nb), du, shots, dout, stream);
 }
 
 void scale_state(aqs_state s, double factor) {

@@ -3,7 +3,9 @@
 qubit, then CZ on alternating nearest-neighbour pairs) on one MI355X.
 
 A step is one simulate() of the whole circuit from |0..0> with the plain
-per-gate HIP kernels (830 gate passes over the 2 GiB state).  The JSON line
+per-gate HIP kernels (830 gate passes over the 2 GiB state: one aqs_apply call
+per gate; a call with the whole list runs many gates per sweep and is reported
+beside it).  The JSON line
 reports gate-applications/s for that path, the HBM roofline of its dominant
 kernel (the one-qubit U3 pass), the compile()-fused form of the same circuit,
 infidelity against a complex128 run of the same circuit, and the FP64 CPU
@@ -31,6 +33,17 @@ N_QUBITS = 28
 DEPTH = 20
 SEED = 2
 HBM_PEAK_GBS = 8000.0
+
+
+def packed_each(lowered):
+    """Every op packed on its own, for the plain per-gate path."""
+    return [hip.PackedOps([o]) for o in lowered]
+
+
+def apply_each(st, packed):
+    """The plain per-gate path: one call, and one kernel pass, per op."""
+    for p in packed:
+        st.apply(p)
 
 
 def log(msg):
@@ -203,12 +216,15 @@ def random20(args, n=20, depth=40, shots=1000):
     st = hip.State(n, hip.C64)
     out = {"qubits": n, "depth": depth, "gates": len(lowered), "shots": shots}
     reps = max(3, args.steps)
-    for label, sch in (("plain", None), ("fused_k5", hip.Schedule(lowered, n, 5)),
+    each, whole = packed_each(lowered), hip.PackedOps(lowered)
+    for label, sch in (("plain", None), ("one_call", None), ("fused_k5", hip.Schedule(lowered, n, 5)),
                        ("tiled", hip.Schedule(lowered, n, mode="tiled"))):
         def run_once():
             st.set_basis(0)
-            if sch is None:
-                st.apply(lowered)
+            if label == "plain":
+                apply_each(st, each)
+            elif label == "one_call":
+                st.apply(whole)
             else:
                 st.apply_schedule(sch)
             return st.sample(u)
@@ -317,10 +333,11 @@ def qft30(args, n=30, seed=30, inverse=False):
         ov = st.inner(ref)
         return max(0.0, 1.0 - abs(ov) ** 2 / (st.norm2() * ref.norm2()))
 
+    each = packed_each(lowered)
     st.gaussian(seed)
     st.sync()
     t0 = time.perf_counter()
-    st.apply(lowered)
+    apply_each(st, each)
     st.sync()
     dt = time.perf_counter() - t0
     out["unfused"] = {"ms": round(1e3 * dt, 2), "gate_apps_per_s": round(len(lowered) / dt, 1),
@@ -419,8 +436,8 @@ def serve_stream(reqs, rate, budget, workers, seed, coalesce=True):
 
 def served(args):
     """Poisson arrivals of mixed-size brickwork requests into the request
-    server (4 workers; compile() fusion per request above 16 qubits, queued
-    requests of at most 16 qubits coalesced into batched launches): p50/p99
+    server (4 workers; runs of ops up to 24 qubits, compile() fusion
+    above, queued requests of at most 16 qubits coalesced into batched launches): p50/p99
     latency (arrival -> sampled indices) and throughput at arrival rates from
     0.7x one worker's capacity up to and past the saturation of all four, and
     at the two highest rates with coalescing off; the same requests run one
@@ -455,15 +472,16 @@ def served(args):
     # per-gate kernels (no fusion, no concurrency), same uniforms; the fused
     # one-worker service time above is on the same requests
     plain = calib
+    plain_each = [packed_each(r["ops"]) for r in plain]
     st_cache = {}
     t0 = time.perf_counter()
     worst_plain = 0.0
-    for r in plain:
+    for r, each in zip(plain, plain_each):
         st = st_cache.get(r["n"])
         if st is None:
             st = st_cache[r["n"]] = hip.State(r["n"], hip.C64)
         st.set_basis(0)
-        st.apply(r["packed"])
+        apply_each(st, each)
         st.sample(r["u"])
     plain_s = time.perf_counter() - t0
     for st in st_cache.values():
@@ -582,9 +600,11 @@ def run(args):
     tuned = st.autotune(reps=3)
     log(f"autotuned one-qubit launch shapes in {time.perf_counter() - t0:.2f} s: {tuned}")
 
+    each = packed_each(lowered)
+
     def step():
         st.set_basis(0)
-        st.apply(lowered)
+        apply_each(st, each)
 
     for _ in range(args.warmup):
         step()
@@ -621,12 +641,28 @@ def run(args):
     ref = hip.State(n, hip.C128)
     ref.set_basis(0)
     ref.apply(ops.lower_all(gates, exact=True))
-    st.set_basis(0)
-    st.apply(lowered)
+    step()
     ov = st.inner(ref)
     n64 = st.norm2()
     infid = max(0.0, 1.0 - abs(ov) ** 2 / n64)
     log(f"infidelity plain c64 vs c128: {infid:.3e}")
+
+    # the same ops in one aqs_apply call: runs in LDS tiles, planned per call
+    whole = hip.PackedOps(lowered)
+    st.set_basis(0)
+    st.apply(whole)
+    st.sync()
+    t0 = time.perf_counter()
+    for _ in range(args.steps):
+        st.set_basis(0)
+        st.apply(whole)
+    st.sync()
+    rdt = (time.perf_counter() - t0) / args.steps
+    ov = st.inner(ref)
+    uncompiled = {"ms_per_step": round(1e3 * rdt, 3), "gate_apps_per_s": round(n_gates / rdt, 1),
+                  "infidelity": max(0.0, 1.0 - abs(ov) ** 2 / st.norm2()),
+                  "speedup_vs_plain": round((dt / args.steps) / rdt, 3)}
+    log(f"uncompiled list in one call: {uncompiled}")
 
     # compile(): fused 5-qubit (and smaller) blocks on the same circuit
     fused = {}
@@ -688,6 +724,7 @@ def run(args):
         "hbm_gbs_per_step": round(alg_bytes / (ms_per_step * 1e-3) / 1e9, 1),
         "infidelity_vs_fp64": infid,
         "roofline": roofline,
+        "uncompiled_one_call": uncompiled,
         "fused": fused,
         "batched": batch,
         "random20": r20,

@@ -97,9 +97,8 @@ inline bool run_takes(const aqs_op& op) { return op.kind != AQS_OP_MATK; }
 // diagonally commute).
 std::vector<RunLaunch> plan_runs(const aqs_op* ops, size_t count, int n, int m, int precision);
 
-// Applies validated ops that run_takes() through runs (runs.hip); returns the
-// number of launches.
-size_t apply_run(aqs_state s, const aqs_op* ops, size_t count);
+// Applies validated ops that run_takes() through runs (runs.hip).
+void apply_run(aqs_state s, const aqs_op* ops, size_t count);
 
 }  // namespace aqs_hip
 

@@ -263,7 +263,7 @@ static int run_tile_qubits(int n, int precision) {
     return n <= 11 ? n : n <= 18 ? 11 : kRunMaxTileC128;
 }
 
-size_t apply_run(aqs_state s, const aqs_op* ops, size_t count) {
+void apply_run(aqs_state s, const aqs_op* ops, size_t count) {
     const int m = run_tile_qubits(s->n, s->precision);
     const std::vector<RunLaunch> launches = plan_runs(ops, count, s->n, m, s->precision);
     for (const RunLaunch& l : launches) {
@@ -281,7 +281,6 @@ size_t apply_run(aqs_state s, const aqs_op* ops, size_t count) {
         else
             launch_run<double2, double>(s, a);
     }
-    return launches.size();
 }
 
 }  // namespace aqs_hip

@@ -5,9 +5,7 @@
 // shot count; its result is the sampled basis indices.  Each worker thread
 // owns a HIP stream (default priority) and runs one request at a time:
 // compile() fusion on the host (aqs_fuse_auto, or aqs_fuse of a fixed
-// width), then |0..0>, the fused passes and sampling on its stream; or, with
-// automatic fusion and at most kRunRequestQubits qubits, the ops as runs
-// (runs.h) without a compilation that is used once.  Gate
+// width), then |0..0>, the fused passes and sampling on its stream.  Gate
 // kernels are deterministic, so a request's result does not depend on what
 // else runs beside it.
 //
@@ -23,7 +21,7 @@
 
 #include "batch.h"
 #include "internal.h"
-#include "runs.h"
+#include "schedule.h"
 #include "serve_core.h"
 
 using namespace aqs_hip;
@@ -44,13 +42,10 @@ size_t state_footprint(int n) {
 // circuits and 1000 shots each fit.
 constexpr size_t kArenaBytes = 96ull << 20;
 
-// A circuit is run once per request, so compiling it pays only when it saves
-// more device time than it takes.  Brickwork depth 40 from a gate list to the
-// final state, compiled / as runs, us: 17 qubits 1810 / 555, 20 qubits 2077 /
-// 768, 22 qubits 2773 / 1308, 24 qubits 5477 / 4522 (depth 10: 803 / 148, 585 /
-// 222, 686 / 341, 1386 / 1192); above, device time (twice as much per
-// qubit) decides, and compiled circuits take less of it.
-constexpr int kRunRequestQubits = 24;
+// Requests of up to this size are compiled to tiles only.  aqs_fuse_auto also
+// builds four block schedules on threads of their own and, at these sizes, nearly
+// always drops them; with several workers they compete for the host.
+constexpr int kTileRequestQubits = 24;
 
 // What the state pool holds for the backend: a request's state or a group arena.
 struct Resident {
@@ -134,23 +129,20 @@ class HipBackend final : public aqs_serve::Backend {
             if (r.cancel.load()) throw ServeError{AQS_ERR_RUNTIME, "request cancelled"};
         };
         aqs_schedule sch = nullptr;
-        bool runs = fuse_qubits_ == 0 && r.n <= kRunRequestQubits;
-        for (const auto& op : r.ops) runs = runs && run_takes(op);
+        bool tiles = r.n >= 10 && r.n <= kTileRequestQubits;
+        for (const auto& op : r.ops) tiles = tiles && op.kind != AQS_OP_MATK;
         try {
-            if (runs)
-                ;
+            if (fuse_qubits_ == 0 && tiles)
+                ck(aqs_fuse_tiled(r.ops.data(), r.ops.size(), r.n, auto_tile_qubits(r.n), &sch));
             else if (fuse_qubits_ == 0)
                 ck(aqs_fuse_auto(r.ops.data(), r.ops.size(), r.n, &sch));
             else
                 ck(aqs_fuse(r.ops.data(), r.ops.size(), r.n, fuse_qubits_, &sch));
-            if (sch) ck(aqs_schedule_info(sch, &r.passes, nullptr));
+            ck(aqs_schedule_info(sch, &r.passes, nullptr));
             stop_if_cancelled();
             ck(aqs_state_set_stream(st, streams_[(size_t)worker]));
             ck(aqs_state_set_basis(st, 0));
-            if (sch)
-                ck(aqs_apply_schedule(st, sch));
-            else
-                ck(guard([&] { r.passes = apply_run(st, r.ops.data(), r.ops.size()); }));
+            ck(aqs_apply_schedule(st, sch));
             stop_if_cancelled();
             r.indices.resize(r.shots);
             if (r.shots) ck(aqs_sample(st, r.u.data(), r.shots, r.indices.data()));

@@ -51,7 +51,6 @@ namespace {
 // 490; 20: 966, 634 / 614 / 601; brickwork depth 20: 14: 148, 102 / 101 / 123;
 // 22: 926, 601 / 456 / 418.
 constexpr int kTileAutoMinQubits = 10, kTileListedMinQubits = 20;
-int auto_tile_qubits(int n) { return n <= 13 ? n : n <= 19 ? 12 : kTileMaxLocal; }
 
 // A phase term: multiply by z where every listed index bit is 1.
 struct Term {
@@ -434,48 +433,37 @@ class Tiler {
     static constexpr double kDenseMinCost = 3.2;
 
     // The 4 local index bits whose ready members cost most, grown from the
-    // first ready members' bits (0: none worth a dense op).
+    // first ready member's bits (0: none worth a dense op).  (Starting from
+    // the first three took twice the host time for the same modelled cost, within
+    // 6%, better or worse.)
     uint64_t best_block(const std::vector<Member>& ms, const std::vector<char>& mdone, uint64_t local) const {
-        uint64_t best = 0;
-        double best_cost = kDenseMinCost;
-        uint64_t nd = 0, dg = 0, tried = 0;
-        int seeds = 0;
-        for (size_t k = 0; k < ms.size() && seeds < 3; ++k) {
+        uint64_t nd = 0, dg = 0;
+        for (size_t k = 0; k < ms.size(); ++k) {
             if (mdone[k]) continue;
             const Member& o = ms[k];
-            if ((o.nd & (nd | dg)) || (o.dg & nd) || !o.fits || !o.nd || __builtin_popcountll(o.nd | o.dg) > 4 ||
-                (o.nd & tried)) {
-                if (!(o.nd & tried)) {
-                    nd |= o.nd;
-                    dg |= o.dg;
-                }
+            if ((o.nd & (nd | dg)) || (o.dg & nd) || !o.fits || !o.nd || __builtin_popcountll(o.nd | o.dg) > 4) {
+                nd |= o.nd;
+                dg |= o.dg;
                 continue;
             }
-            ++seeds;
             uint64_t set = o.nd | o.dg;
-            double c = 0;
+            double c = __builtin_popcountll(set) == 4 ? capture(ms, mdone, set, nullptr) : 0;
             while (__builtin_popcountll(set) < 4) {
                 uint64_t pick = 0;
-                double pc = -1;
+                c = -1;
                 for (uint64_t rest = local & ~set; rest; rest &= rest - 1) {
                     const uint64_t b = rest & (0 - rest);
                     const double bc = capture(ms, mdone, set | b, nullptr);
-                    if (bc > pc) {
-                        pc = bc;
+                    if (bc > c) {
+                        c = bc;
                         pick = b;
                     }
                 }
                 set |= pick;
-                c = pc;
             }
-            tried |= set;
-            if (c == 0) c = capture(ms, mdone, set, nullptr);
-            if (c > best_cost) {
-                best_cost = c;
-                best = set;
-            }
+            return c > kDenseMinCost ? set : 0;
         }
-        return best;
+        return 0;
     }
 
     // Applies a member to the rows of a 16 x 16 matrix whose index bit i is
@@ -1001,6 +989,21 @@ bool diag_rides_block(const aqs_schedule_s* sch, size_t p) {
     return false;
 }
 
+// Below 20 qubits a pass is bound by its launch and by the chain of ops in
+// its few workgroups, not by sweeps.  Fitted in us: a tile pass 9 and 6 per unit
+// of its modelled work beyond the sweep (random layers, 15 / 17 / 19 qubits
+// depth 40: 245 / 371 / 456 modelled, 245 / 364 / 464 measured; brickwork depth 20,
+// 14 / 18 qubits: 95 / 178, 101 / 177; ansatz, 16 qubits depth 60: 1098, 1149); a
+// block pass 4.5 up to 17 qubits, 5.8 above (343 / 442 / 643, 148 / 235, 1052
+// measured).
+double small_tiles_us(const aqs_schedule_s* sch) {
+    const double passes = (double)sch->passes.size();
+    return 9.0 * passes + 6.0 * std::max(0.0, schedule_cost(sch) - 1.03 * passes);
+}
+double small_blocks_us(const aqs_schedule_s* sch) {
+    return (sch->n <= 17 ? 4.5 : 5.8) * (double)sch->passes.size();
+}
+
 }  // namespace
 
 // Operand A of v_mfma_f32_32x32x16_bf16 for each unitary, [plane][real or
@@ -1039,6 +1042,8 @@ std::vector<uint16_t> aqs_hip::pack_dense(const std::vector<double>& dense) {
     }
     return out;
 }
+
+int aqs_hip::auto_tile_qubits(int n) { return n <= 13 ? n : n <= 19 ? 12 : kTileMaxLocal; }
 
 double aqs_hip::schedule_cost(const aqs_schedule_s* sch) {
     double c = 0;
@@ -1119,7 +1124,8 @@ aqs_status aqs_fuse_auto(const aqs_op* ops, size_t count, int nqubits, aqs_sched
         set_error(terr);
         return tst;
     }
-    const bool keep_tiled = schedule_cost(tiled) < schedule_cost(blocks);
+    const bool keep_tiled = nqubits < kTileListedMinQubits ? small_tiles_us(tiled) < small_blocks_us(blocks)
+                                                           : schedule_cost(tiled) < schedule_cost(blocks);
     if (keep_tiled && nqubits < kTileListedMinQubits) {
         blocks->tile_form = tiled;
         *out = blocks;

@@ -1013,32 +1013,36 @@ double small_blocks_us(const aqs_schedule_s* sch) {
 std::vector<uint16_t> aqs_hip::pack_dense(const std::vector<double>& dense) {
     const size_t count = dense.size() / kDenseDoubles;
     std::vector<uint16_t> out(count * kDenseOperand);
-    auto bf16 = [](double v, double& back) {  // to nearest, ties to even
-        const float f = (float)v;
-        uint32_t w;
-        std::memcpy(&w, &f, 4);
-        w += 0x7FFFu + ((w >> 16) & 1u);
-        w &= 0xFFFF0000u;
-        float r;
-        std::memcpy(&r, &w, 4);
-        back = r;
-        return (uint16_t)(w >> 16);
+    auto split = [](double v, uint16_t (&w)[3]) {  // to nearest, ties to even, then the rest
+        for (uint16_t& x : w) {
+            const float f = (float)v;
+            uint32_t b;
+            std::memcpy(&b, &f, 4);
+            b = (b + 0x7FFFu + ((b >> 16) & 1u)) & 0xFFFF0000u;
+            x = (uint16_t)(b >> 16);
+            float r;
+            std::memcpy(&r, &b, 4);
+            v -= r;
+        }
     };
     for (size_t c = 0; c < count; ++c) {
         const double* u = dense.data() + c * kDenseDoubles;
-        for (int s = 0; s < 2; ++s)
-            for (int l = 0; l < 64; ++l)
-                for (int j = 0; j < 8; ++j) {
-                    const int row = l % 32, g = row / 8, h = (row / 4) % 2, e = row % 4;
-                    const int amp = 8 * h + 4 * (g / 2) + e, col = 8 * (l / 32) + j;
-                    const double re = u[2 * (16 * amp + col)], im = u[2 * (16 * amp + col) + 1];
-                    double v = g % 2 == 0 ? (s == 0 ? re : -im) : (s == 0 ? im : re);
-                    for (int p = 0; p < 3; ++p) {
-                        double back;
-                        out[c * kDenseOperand + (size_t)(((2 * p + s) * 64 + l) * 8 + j)] = bf16(v, back);
-                        v -= back;
-                    }
+        uint16_t* o = out.data() + c * kDenseOperand;
+        for (int amp = 0; amp < 16; ++amp)
+            for (int col = 0; col < 16; ++col) {
+                uint16_t re[3], im[3];
+                split(u[2 * (16 * amp + col)], re);
+                split(u[2 * (16 * amp + col) + 1], im);
+                // this entry's place in the rows of the real and of the imaginary part
+                const int row = 16 * ((amp >> 2) & 1) + 4 * (amp >> 3) + (amp & 3);
+                const int at = 8 * (row + 32 * (col >> 3)) + (col & 7), at_im = at + 64;
+                for (int p = 0; p < 3; ++p) {
+                    uint16_t* k = o + 1024 * p;  // real columns, then imaginary ones
+                    k[at] = k[512 + at_im] = re[p];
+                    k[at_im] = im[p];
+                    k[512 + at] = im[p] ^ 0x8000u;
                 }
+            }
     }
     return out;
 }

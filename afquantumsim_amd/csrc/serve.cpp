@@ -45,7 +45,7 @@ constexpr size_t kArenaBytes = 96ull << 20;
 // Requests of up to this size are compiled to tiles only.  aqs_fuse_auto also
 // builds four block schedules on threads of their own and, at these sizes, nearly
 // always drops them; with several workers they compete for the host.
-constexpr int kTileRequestQubits = 24;
+constexpr int kTileRequestQubits = 19;
 
 // What the state pool holds for the backend: a request's state or a group arena.
 struct Resident {
